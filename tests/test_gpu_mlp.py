@@ -102,3 +102,22 @@ def test_training_reduces_loss():
     _, l1 = net.gradient(F, t)
     print(f"[train] loss {l0:.4e} -> {l1:.4e}", flush=True)
     assert l1 < 0.2 * l0
+
+
+@pytest.mark.parametrize("n,copies", [(1, 2), (1, 64), (15, 4), (16, 8), (17, 2), (31, 2), (33, 4), (127, 2), (129, 8),
+                                      (500, 16), (4099, 8)])
+def test_gradient_does_not_depend_on_where_a_row_sits(n, copies):
+    """The mean gradient of n rows is that of the same rows repeated a power of
+    two times: each row's BF16 values scale exactly, only the FP32 sums are
+    taken in another order.  The repeats put every row into other tiles, waves,
+    workgroups and (past 32,768 rows) passes of the gradient kernel.  At most
+    ~600 FP32 additions follow one another (6e-8 each): 1e-4 of the norm leaves
+    a factor of three for cancellation."""
+    F, t = _data(n, 11)
+    net = Lr.MLP(seed=3)
+    g1, l1 = net.gradient(F, t)
+    g2, l2 = net.gradient(np.tile(F, (copies, 1)), np.tile(t, copies))
+    assert abs(l1 - l2) <= 1e-4 * l1
+    a, b = Lr.unpack(g1), Lr.unpack(g2)
+    for k in a:
+        assert np.linalg.norm(a[k] - b[k]) <= 1e-4 * np.linalg.norm(a[k]) + 1e-12, k
