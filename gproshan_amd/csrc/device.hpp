@@ -28,13 +28,14 @@ struct DeviceMesh {
 	uint8_t *closed = nullptr; // 1 when the fan of v is closed (link = first m entries)
 	float h = 1.f, inv_h = 1.f;
 	MasterLayout *master[2] = { nullptr, nullptr };   // vertex-major slot tables (FP32, FP64), built on demand
+	uint32_t *link8 = nullptr; // first 8 link entries of each vertex (levels.hip), built on demand
 };
 
 // Uploads the fan tables and FP64 positions of m once (m.dev caches them).
 int upload_mesh(Che &m);
 
-// Replayed launch sequences (sweeps, BFS levels, patch launches, the batch)
-// run from hipGraphs unless the environment sets
+// Replayed launch sequences (sweeps, patch launches, the batch) run from
+// hipGraphs unless the environment sets
 // GPROSHAN_AMD_GRAPHS=0: then the same kernels are launched one by one on the
 // stream, with the same results (a profiler that cannot follow graph replays
 // traces these).

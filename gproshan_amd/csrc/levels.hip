@@ -3,21 +3,20 @@
 
 #include <algorithm>
 #include <memory>
+#include <mutex>
 #include <type_traits>
 
 #include "gp_internal.hpp"
 
 namespace gp {
 
-// Frontier BFS state: launch k expands the frontier queue[fa, fb) of level L
-// (slot (k-1) & 3 advanced by the count cnt[(k-1) & 3] of the vertices the
-// previous launch appended), appending the vertices it lowers to level L + 1
-// after fb through cnt[k & 3].
-struct LSlot {
-	uint32_t L, fa, fb, done, fresh, pad0, pad1, pad2;
-};
+// BFS state: launch k expands the cnt[(k - 1) & 3] vertices queued by the one
+// before (queue half k & 1) and queues the next ones in the other half through
+// cnt[k & 3].  serial numbers the launches over the life of the state (the marks
+// that keep a vertex from being queued twice by one launch); a launch reads it
+// from slot (k - 1) & 3 and workgroup 0 publishes the next in slot k & 3.
 struct LevelState {
-	LSlot slot[4];
+	uint32_t serial[4];
 	uint32_t cnt[4];
 	uint32_t done, launches, max_level, pad;
 };
@@ -33,100 +32,171 @@ __global__ void k_lv_clear(uint32_t *level, uint32_t n)
 	for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) level[v] = GP_NIL;
 }
 
-// Seeds the frontier BFS: sources src[first, ns) get level 0 and form the
-// frontier.
+// Seeds the BFS: sources src[first, ns) get level 0 and form the frontier of
+// launch 0.
 __global__ void k_lv_seed(const uint32_t *src, uint32_t first, uint32_t ns, uint32_t *level, uint32_t *queue,
-                          LevelState *ls)
+                          LevelState *ls, uint32_t fresh)
 {
 	for (uint32_t q = first + threadIdx.x; q < ns; q += blockDim.x) {
 		level[src[q]] = 0;
 		queue[q - first] = src[q];
 	}
 	if (threadIdx.x == 0) {
-		uint32_t *w = (uint32_t *) ls;
-		for (uint32_t q = 0; q < sizeof(LevelState) / 4; q++) w[q] = 0;
-		ls->slot[3].L = 0; ls->slot[3].fa = 0; ls->slot[3].fb = ns - first; ls->slot[3].fresh = 1;
-		ls->slot[3].done = ns > first ? 0u : 1u;
-		ls->done = ls->slot[3].done;
+		uint32_t s = 0;
+		if (!fresh)
+			for (uint32_t q = 0; q < 4; q++) s = max(s, ls->serial[q]);
+		for (uint32_t q = 0; q < 4; q++) { ls->serial[q] = s; ls->cnt[q] = 0; }
+		ls->cnt[3] = ns - first;
+		ls->launches = ls->max_level = ls->pad = 0;
+		ls->done = ns > first ? 0u : 1u;
 	}
 }
 
-// One BFS level over all workgroups.  A neighbour whose level drops to L + 1
-// (atomicMin: exactly one thread sees it drop) is appended once.  A lane
-// issues the atomics of LVU fan entries back to back (slots past its fan
-// apply the no-op minimum NIL to its own vertex), so one level costs one
-// atomic round trip per LVU entries, not one per entry; the appends of a wave
-// take one counter atomic per pass (ballot per entry slot).
-constexpr uint32_t LVU = 8;
+// First 8 link entries of each vertex in 32 bytes (NIL past the link; LONG_LINK
+// on entry 7 when the link goes on in the fan table).
+constexpr uint32_t LONG_LINK = 0x80000000u, LINK_ROW = 8;
 
-__global__ __launch_bounds__(256) void k_lv_step(const uint32_t *fan_off, const uint32_t *fan, uint32_t *level,
-                                                 uint32_t *queue, LevelState *ls, uint32_t k4)
+__global__ void k_link8(const uint32_t *fan_off, const uint32_t *fan, const uint8_t *closed, uint32_t nv,
+                        uint32_t *link8)
 {
+	const size_t n8 = (size_t) nv * LINK_ROW;   // vertex ids stay below 2^31 (build_che)
+	for (size_t q = blockIdx.x * blockDim.x + threadIdx.x; q < n8; q += gridDim.x * blockDim.x) {
+		const uint32_t v = (uint32_t) (q / LINK_ROW), k = (uint32_t) (q % LINK_ROW);
+		const uint32_t s = fan_off[v], c = fan_off[v + 1] - s;
+		const uint32_t n = (c && closed[v]) ? c - 1 : c;
+		uint32_t id = k < n ? fan[s + k] : GP_NIL;
+		if (k == LINK_ROW - 1 && n > LINK_ROW) id |= LONG_LINK;
+		link8[q] = id;
+	}
+}
+
+// LV_DEPTH levels of the frontier in one launch.  A workgroup takes up to
+// LV_CHUNK queued vertices into LDS and pushes level + 1 to their links, eight
+// lanes a vertex; a vertex whose level dropped (exactly one atomicMin sees it
+// drop) is expanded next by the workgroup that lowered it, from LDS, and the
+// vertices of the last depth form the next launch's frontier.  A drop is always
+// expanded, here or by a later launch, so the BFS ends at the hop distances in
+// any order; as all workgroups start from one level, each vertex is lowered
+// once but for the seams between workgroups.
+//
+// Bound by the round trips of a level.  A lane asks for its neighbour's own
+// link with the atomic on its level, so the next level starts from LDS and a
+// level costs one round trip (~1.3 us) instead of a launch and four (state,
+// queue, fan offsets, fan, atomic).  1M-vertex mesh, one source: 992 launches
+// of 5.9 us before (5.8 ms), 58 of 22 us now (1.29 ms); 201k vertices, 16
+// sources: 1.23 -> 0.31 ms; 10k vertices: 0.39 -> 0.13 ms.  24 or 32
+// levels a launch and 64, 128 or 512 threads were no faster on all three.
+// (Running spatial tiles of 1,024 vertices to their end in LDS instead needs
+// ~200 launches of 50-120 us on the 1M mesh: a tile entered from one side first
+// is corrected again and again.)
+constexpr uint32_t LV_T = 256, LV_CHUNK = LV_T / LINK_ROW, LV_DEPTH = 16, LV_Q = 512, LV_SPREAD = 512;
+
+struct LvArgs {
+	const uint32_t *link8, *fan_off, *fan;
+	uint32_t *level, *queue, *mark;
+	LevelState *ls;
+	uint32_t nv;
+};
+
+__global__ __launch_bounds__(LV_T) void k_lv_step(LvArgs a, uint32_t k4)
+{
+	__shared__ uint32_t s_link[2][LV_Q][LINK_ROW], s_id[2][LV_Q], s_lev[2][LV_Q], s_n[3];
+	LevelState *ls = a.ls;
+	const uint32_t tid = threadIdx.x, lane = tid & 63u, slot = tid % LINK_ROW, group = tid / LINK_ROW;
 	const uint32_t kp = (k4 + 3u) & 3u;
-	const LSlot prev = ls->slot[kp];
-	const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-	if (prev.done) {
-		if (lead) ls->slot[k4] = prev;
-		return;
-	}
-	LSlot cur = prev;
-	cur.fresh = 0;
-	if (!prev.fresh) {
-		const uint32_t c = ls->cnt[kp];
-		cur.L = prev.L + 1; cur.fa = prev.fb; cur.fb = prev.fb + c; cur.done = c == 0;
-	}
-	if (lead) {
-		ls->slot[k4] = cur;
+	const uint32_t n = ls->cnt[kp], serial = ls->serial[kp] + 1;
+	const uint32_t *q_in = a.queue + (size_t) (k4 & 1u) * a.nv;
+	uint32_t *q_out = a.queue + (size_t) ((k4 + 1u) & 1u) * a.nv;
+	if (blockIdx.x == 0 && tid == 0) {
+		ls->serial[k4] = serial;
 		ls->cnt[(k4 + 1u) & 3u] = 0;
-		ls->launches = ls->launches + 1;
-		if (cur.done) ls->done = 1;
+		if (n == 0) ls->done = 1;
+		else ls->launches = ls->launches + 1;
 	}
-	if (cur.done) return;
-	const uint32_t lane = threadIdx.x & 63u;
-	const unsigned long long below = (1ull << lane) - 1ull;
-	const uint32_t nl1 = cur.L + 1;
-	const uint32_t stride = gridDim.x * blockDim.x;
-	// Wave-uniform loops: every lane of a wave runs the same iterations (the
-	// ballots and the shuffle below need them all).
-	for (uint32_t b = cur.fa + (blockIdx.x * blockDim.x + (threadIdx.x & ~63u)); b < cur.fb; b += stride) {
-		const uint32_t idx = b + lane;
-		const bool act = idx < cur.fb;
-		const uint32_t u = act ? queue[idx] : 0u;
-		const uint32_t e0 = act ? fan_off[u] : 0u, e1 = act ? fan_off[u + 1] : 0u;
-		const uint32_t len = e1 - e0;
-		uint32_t mx = len;
-		for (uint32_t o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t) __shfl_xor(mx, o));
-		for (uint32_t eb = 0; eb < mx; eb += LVU) {
-			uint32_t w[LVU];
-			uint32_t app = 0;
-			if (eb < len) {
-#pragma unroll
-				for (uint32_t k = 0; k < LVU; k++) w[k] = fan[min(e0 + eb + k, e1 - 1u)];
-#pragma unroll
-				for (uint32_t k = 0; k < LVU; k++) {
-					const bool ok = eb + k < len;
-					const uint32_t old = atomicMin(&level[ok ? w[k] : u], ok ? nl1 : GP_NIL);
-					app |= (ok && old > nl1) ? (1u << k) : 0u;
-				}
-			}
-			unsigned long long m[LVU];
-			uint32_t tot = 0;
-#pragma unroll
-			for (uint32_t k = 0; k < LVU; k++) {
-				m[k] = __ballot((app >> k) & 1u);
-				tot += (uint32_t) __popcll(m[k]);
-			}
-			if (tot) {
-				uint32_t base = 0;
-				if (lane == 0) base = atomicAdd(&ls->cnt[k4], tot);
-				base = cur.fb + __shfl(base, 0);
-#pragma unroll
-				for (uint32_t k = 0; k < LVU; k++) {
-					if ((app >> k) & 1u) queue[base + (uint32_t) __popcll(m[k] & below)] = w[k];
-					base += (uint32_t) __popcll(m[k]);
-				}
+	// Vertex w to the next launch's frontier (every lane of the wave calls).
+	auto queue_next = [&](bool want, uint32_t w) {
+		const bool first = want && atomicExch(&a.mark[w], serial) != serial;
+		const unsigned long long m = __ballot(first);
+		if (!m) return;
+		uint32_t base = 0;
+		if (lane == 0) base = atomicAdd(&ls->cnt[k4], (uint32_t) __popcll(m));
+		base = __shfl(base, 0);
+		if (first) q_out[base + (uint32_t) __popcll(m & ((1ull << lane) - 1ull))] = w;
+	};
+	// A short frontier is spread over LV_SPREAD workgroups, one vertex each if
+	// need be: the lists stay short (a 16-source seed by one workgroup: 190 us).
+	const uint32_t chunk = max(1u, min(LV_CHUNK, n / LV_SPREAD));
+	for (uint32_t c0 = blockIdx.x * chunk; c0 < n; c0 += gridDim.x * chunk) {
+		if (tid == 0) { s_n[0] = min(chunk, n - c0); s_n[1] = 0; s_n[2] = 0; }
+		{
+			const uint32_t i = c0 + group;
+			if (group < chunk && i < n) {
+				const uint32_t v = q_in[i];
+				s_link[0][group][slot] = a.link8[(size_t) v * LINK_ROW + slot];
+				if (slot == 0) { s_id[0][group] = v; s_lev[0][group] = a.level[v]; }
 			}
 		}
+		__syncthreads();
+		for (uint32_t d = 0;; d++) {
+			const uint32_t cur = d & 1u, nq = s_n[d % 3u];
+			if (nq == 0) break;
+			const bool last = d + 1 == LV_DEPTH;
+			if (tid == 0) s_n[(d + 2) % 3u] = 0;   // read at depth d - 1, counted from depth d + 1
+			for (uint32_t b = 0; b < nq; b += LV_T / LINK_ROW) {
+				const uint32_t i = b + group;
+				uint32_t w = i < nq ? s_link[cur][i][slot] : GP_NIL;
+				const bool more = w != GP_NIL && (w & LONG_LINK);
+				if (w != GP_NIL) w &= ~LONG_LINK;
+				const uint32_t l1 = i < nq ? s_lev[cur][i] + 1 : 0u;
+				bool won = false;
+				uint4 r0 = make_uint4(0, 0, 0, 0), r1 = r0;
+				if (w != GP_NIL) {
+					const uint4 *row = (const uint4 *) (a.link8 + (size_t) w * LINK_ROW);
+					r0 = row[0];
+					r1 = row[1];
+					won = atomicMin(&a.level[w], l1) > l1;
+				}
+				bool out = won && last;
+				// Room in the next depth's list: one LDS counter add per wave.
+				const unsigned long long m = last ? 0ull : __ballot(won);
+				uint32_t at = 0;
+				if (m) {
+					if (lane == 0) at = atomicAdd(&s_n[(d + 1) % 3u], (uint32_t) __popcll(m));
+					at = __shfl(at, 0) + (uint32_t) __popcll(m & ((1ull << lane) - 1ull));
+				}
+				if (won && !last) {
+					if (at < LV_Q) {
+						*(uint4 *) &s_link[cur ^ 1u][at][0] = r0;
+						*(uint4 *) &s_link[cur ^ 1u][at][4] = r1;
+						s_id[cur ^ 1u][at] = w;
+						s_lev[cur ^ 1u][at] = l1;
+					} else {
+						out = true;   // no room: the next launch expands it
+					}
+				}
+				queue_next(out, w);
+				if (__ballot(more)) {
+					// Links longer than a row: lane 7 of the vertex walks the
+					// rest in the fan table.
+					uint32_t e = 0, e1 = 0;
+					if (more) {
+						const uint32_t v = s_id[cur][i];
+						e = a.fan_off[v] + LINK_ROW;
+						e1 = a.fan_off[v + 1];
+					}
+					while (__ballot(e < e1)) {
+						const bool act = e < e1;
+						const uint32_t u = act ? a.fan[e] : 0u;
+						queue_next(act && atomicMin(&a.level[u], l1) > l1, u);
+						e++;
+					}
+				}
+			}
+			__syncthreads();
+			if (tid == 0) s_n[(d + 1) % 3u] = last ? 0u : min(s_n[(d + 1) % 3u], LV_Q);
+			__syncthreads();
+		}
+		__syncthreads();
 	}
 }
 
@@ -306,25 +376,45 @@ __global__ __launch_bounds__(1024) void k_exclusive_scan(const uint32_t *in, uin
 	if (threadIdx.x == 0) out[n] = carry;
 }
 
-constexpr uint32_t LV = 32;   // level launches per graph replay
-
 Levels::~Levels()
 {
-	for (void *p : { (void *) level, (void *) queue, (void *) hist, (void *) sorted, (void *) limits, (void *) nl,
-	                 (void *) ls, (void *) cslots, (void *) coff })
+	for (void *p : { (void *) level, (void *) queue, (void *) mark, (void *) hist, (void *) sorted, (void *) limits,
+	                 (void *) nl, (void *) ls, (void *) cslots, (void *) coff })
 		(void) hipFree(p);
 	if (h_ls) (void) hipHostFree(h_ls);
-	if (graph) (void) hipGraphExecDestroy(graph);
 	for (hipEvent_t e : ev)
 		if (e) (void) hipEventDestroy(e);
 }
 
-int Levels::create(const DeviceMesh *mesh, hipStream_t s)
+static uint32_t fill_grid(uint32_t n) { return std::max<uint32_t>(1, std::min<uint32_t>(2048, (n + 255) / 256)); }
+
+// The mesh's link rows, built once on first use (several threads may ask).
+static int link_rows(DeviceMesh *dm)
+{
+	static std::mutex mu;
+	std::lock_guard<std::mutex> lock(mu);
+	if (dm->link8) return GP_OK;
+	uint32_t *p = nullptr;
+	if (hipMalloc(&p, 4ull * LINK_ROW * dm->nv) != hipSuccess)
+		return fail(GP_ERR_NOMEM, "levels: device allocation failed");
+	k_link8<<<fill_grid(dm->nv), 256>>>(dm->fan_off, dm->fan, dm->closed, dm->nv, p);
+	const hipError_t e = hipGetLastError() != hipSuccess ? hipErrorUnknown : hipDeviceSynchronize();
+	if (e != hipSuccess) {
+		(void) hipFree(p);
+		return fail(GP_ERR_HIP, "levels: link rows: %s", hipGetErrorString(e));
+	}
+	dm->link8 = p;
+	return GP_OK;
+}
+
+int Levels::create(DeviceMesh *mesh, hipStream_t s)
 {
 	dm = mesh;
 	nv = mesh->nv;
 	stream = s;
-	if (hipMalloc(&level, 4ull * nv) != hipSuccess || hipMalloc(&queue, 4ull * nv) != hipSuccess ||
+	if (int rc = link_rows(mesh)) return rc;
+	if (hipMalloc(&level, 4ull * nv) != hipSuccess || hipMalloc(&queue, 8ull * nv) != hipSuccess ||
+	    hipMalloc(&mark, 4ull * nv) != hipSuccess ||
 	    hipMalloc(&hist, 4ull * ((size_t) nv * LEVEL_KEYS + 1)) != hipSuccess ||
 	    hipMalloc(&sorted, 4ull * nv) != hipSuccess || hipMalloc(&cslots, 4ull * (nchunks() + 1)) != hipSuccess ||
 	    hipMalloc(&coff, 4ull * (nchunks() + 1)) != hipSuccess ||
@@ -333,59 +423,46 @@ int Levels::create(const DeviceMesh *mesh, hipStream_t s)
 		return fail(GP_ERR_NOMEM, "levels: device allocation failed");
 	GP_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
 	GP_HIP(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
-	// Enough workgroups for a frontier of 64k vertices per pass.
-	// One wave per workgroup, as the sweeps.
-	const uint32_t grid = std::max<uint32_t>(1, std::min<uint32_t>(1024, (nv + 63) / 64));
-	lv_grid = grid;
-	if (!graphs_enabled()) return GP_OK;
-	const uint32_t *fo = dm->fan_off, *fa = dm->fan;
-	const uint32_t k4s[4] = { 0, 1, 2, 3 };
-	GraphChain gc;
-	for (uint32_t q = 0; q < LV; q++) {
-		void *args[] = { (void *) &fo, (void *) &fa, (void *) &level, (void *) &queue, (void *) &ls,
-		                 (void *) &k4s[q & 3u] };
-		gc.add((const void *) k_lv_step, dim3(grid), dim3(64), args);
-	}
-	const hipError_t e = gc.instantiate(&graph);
-	if (e != hipSuccess) return fail(GP_ERR_HIP, "levels graph: %s", hipGetErrorString(e));
+	k_lv_zero<<<fill_grid(nv), 256, 0, stream>>>(mark, nv);
+	GP_HIP(hipGetLastError());
+	// One workgroup per LV_CHUNK frontier vertices; frontiers past the grid loop.
+	lv_grid = std::max<uint32_t>(1, std::min<uint32_t>(1024, (nv + LV_CHUNK - 1) / LV_CHUNK));
+	fresh = true;
 	return GP_OK;
 }
-
-static uint32_t fill_grid(uint32_t n) { return std::max<uint32_t>(1, std::min<uint32_t>(2048, (n + 255) / 256)); }
 
 void Levels::clear() { k_lv_clear<<<fill_grid(nv), 256, 0, stream>>>(level, nv); }
 
 void Levels::seed(const uint32_t *d_src, uint32_t first, uint32_t ns)
 {
-	k_lv_seed<<<1, 256, 0, stream>>>(d_src, first, ns, level, queue, ls);
+	k_lv_seed<<<1, 256, 0, stream>>>(d_src, first, ns, level, queue, ls, fresh ? 1u : 0u);
+	fresh = false;
 }
 
-// Replays until the state reports done, two in flight: each replay is
-// followed by a kernel that writes the state into its pinned snapshot and an
-// event; the host waits for the older replay while the newer one runs (a
-// replay queued behind the one that finishes meets done slots and returns at
-// once).
+// Launches in rounds of LV until the state reports done, two rounds in flight:
+// each round is followed by a kernel that writes the state into its pinned
+// snapshot and an event; the host waits for the older round while the newer one
+// runs (a round queued behind the one that finishes finds nothing queued).  Few
+// and long launches: one by one on the stream, no graph to build.
+constexpr uint32_t LV = 4;   // a multiple of 4 (the state slots)
+
 int Levels::expand()
 {
 	GP_HIP(hipGetLastError());
-	auto replay = [&](uint32_t s) -> int {
-		if (graph) {
-			GP_HIP(hipGraphLaunch(graph, stream));
-		} else {
-			for (uint32_t q = 0; q < LV; q++)
-				k_lv_step<<<lv_grid, 64, 0, stream>>>(dm->fan_off, dm->fan, level, queue, ls, q & 3u);
-		}
+	const LvArgs a{ dm->link8, dm->fan_off, dm->fan, level, queue, mark, ls, nv };
+	auto round = [&](uint32_t s) -> int {
+		for (uint32_t q = 0; q < LV; q++) k_lv_step<<<lv_grid, LV_T, 0, stream>>>(a, q & 3u);
 		snapshot(ls, h_ls + s, stream);
 		GP_HIP(hipGetLastError());
 		GP_HIP(hipEventRecord(ev[s], stream));
 		return GP_OK;
 	};
-	int rc = replay(0);
+	int rc = round(0);
 	if (rc) return rc;
 	for (uint32_t reps = 0, cur = 0;; reps++, cur ^= 1u) {
-		// Every replay but an empty one lowers at least one vertex.
+		// Every launch but the last lowers at least one vertex.
 		if (reps > nv / LV + 2) return fail(GP_ERR_KERNEL, "levels: BFS did not finish");
-		if ((rc = replay(cur ^ 1u))) return rc;
+		if ((rc = round(cur ^ 1u))) return rc;
 		GP_HIP(hipEventSynchronize(ev[cur]));
 		if (h_ls[cur].done) break;
 	}

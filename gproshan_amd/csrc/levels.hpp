@@ -1,14 +1,14 @@
 // Multi-source BFS levels on the device and the vertices sorted by level (the
 // rings of parallel_toplesets_propagation, che::compute_toplesets,
-// src/che.cpp:546-593, as sets).  A frontier BFS over all workgroups (one
-// launch per level, replayed from a graph, the host polling a done
+// src/che.cpp:546-593, as sets).  A frontier BFS over all workgroups (each
+// launch takes the frontier LV_DEPTH levels further, the host polling a done
 // flag) lowers the levels from the seeded sources, stopping where the levels
-// are already as low -- so seeding one more source into existing levels
-// updates them incrementally -- and a counting sort by level and, inside a
-// level, by slot count (longest fans first) rebuilds sorted[], limits and the
-// slot rows of each 64-position chunk.  The order inside a ring is not the
-// reference's discovery order (the window sweeps relax whole rings, so it
-// changes no value).
+// are already as low -- so seeding one more source into existing levels updates
+// them incrementally -- and a counting sort by level and, inside a level, by
+// slot count (longest fans first) rebuilds sorted[], limits and the slot rows
+// of each 64-position chunk.  The order inside a ring is not the reference's
+// discovery order (the window sweeps relax whole rings, so it changes no
+// value).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -24,7 +24,10 @@ constexpr uint32_t LEVEL_KEYS = 8;   // slot classes per level in the sort key
 struct Levels {
 	uint32_t nv = 0;
 	uint32_t *level = nullptr;    // [nv], NIL = unreached
-	uint32_t *queue = nullptr;    // [nv]
+	uint32_t *queue = nullptr;    // [2][nv] frontier of this launch and the next
+	uint32_t *mark = nullptr;     // [nv] number of the last launch that queued the vertex
+	uint32_t lv_grid = 1;
+	bool fresh = true;            // the state has not been seeded yet
 	uint32_t *hist = nullptr;     // [nv * LEVEL_KEYS + 1]  key counts, then cursors
 	uint32_t *sorted = nullptr;   // [nv]   vertices by level, longest fans first in a level
 	uint32_t *limits = nullptr;   // [nv + 2]
@@ -33,16 +36,14 @@ struct Levels {
 	uint32_t *coff = nullptr;     // [nchunks() + 1] their exclusive prefix (chunk c at row coff[c])
 	LevelState *ls = nullptr, *h_ls = nullptr;   // h_ls: two pinned snapshots
 	hipEvent_t ev[2] = { nullptr, nullptr };
-	hipGraphExec_t graph = nullptr;   // null when graphs are disabled
-	uint32_t lv_grid = 1;
 	hipStream_t stream = nullptr;   // borrowed
-	const DeviceMesh *dm = nullptr;
+	DeviceMesh *dm = nullptr;
 
 	Levels() = default;
 	Levels(const Levels &) = delete;
 	Levels &operator=(const Levels &) = delete;
 	~Levels();
-	int create(const DeviceMesh *mesh, hipStream_t s);
+	int create(DeviceMesh *mesh, hipStream_t s);
 	void clear();                                               // every level unreached
 	void seed(const uint32_t *d_src, uint32_t first, uint32_t ns);   // d_src[first, ns) to level 0
 	int expand();                                               // BFS to completion

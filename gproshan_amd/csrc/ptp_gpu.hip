@@ -59,6 +59,7 @@ void device_mesh_free(DeviceMesh *d)
 	(void) hipFree(d->closed);
 	delete d->master[0];
 	delete d->master[1];
+	(void) hipFree(d->link8);
 	delete d;
 }
 

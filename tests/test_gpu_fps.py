@@ -62,3 +62,24 @@ def test_fps_errors_and_edges():
     assert s.tolist() == [0, 1] and r == np.inf
     s, r, _ = P.farthest_point_sampling_ptp_gpu(C, [0], 10 ** 9)  # V/2 in all
     assert len(s) == len(xyz) // 2 and len(set(s.tolist())) == len(s)
+
+
+@pytest.mark.parametrize("name,gen,init,add", [
+    # A hub of 48 neighbours: a link longer than a link row.
+    ("hub48", lambda: G.polar_disk(9, 48, 5), [0], 4),
+    ("hub48_rim", lambda: G.polar_disk(9, 48, 5), [300], 4),
+    # A first frontier of more vertices than one pass of the grid takes.
+    ("wide_front", lambda: G.height_field(200, 6), list(range(0, 35000)), 2),
+    # Frontiers of one vertex, a full chunk less and more one, over many depths.
+    ("strip31", lambda: G.height_field_rect(31, 400, 7), [0], 3),
+    ("strip33_31src", lambda: G.height_field_rect(33, 300, 8), list(range(1, 63, 2)), 3),
+    ("strip33_33src", lambda: G.height_field_rect(33, 300, 8), list(range(1, 67, 2)), 3),
+], ids=lambda x: x if isinstance(x, str) else "")
+def test_fps_levels_at_the_edges_of_the_bfs(name, gen, init, add, oracle):
+    """The rounds run on levels lowered from each new sample: a wrong or stale
+    level changes a ring, hence the samples."""
+    xyz, f = gen()
+    n = len(init) + add
+    ref, rref = oracle.Mesh(xyz, f).fps(init, n, 0.0)
+    got, r, _ = P.farthest_point_sampling_ptp_gpu(P.che(xyz, f), init, n, precision=L.PREC_F64)
+    assert got.tolist() == ref.tolist() and r == rref
