@@ -27,7 +27,7 @@ struct gp_che {
 	}
 
 static int plan_create_any(gp_che *mesh, const uint32_t *sources, uint32_t n_sources, const double *dhat,
-                           const gp_ptp_opts &o, gp_plan **out);
+                           const gp_ptp_opts &o, gp_plan **out, bool want_order = false);
 
 extern "C" {
 
@@ -297,11 +297,15 @@ int gp_ptp(gp_che *mesh, const uint32_t *sources, uint32_t n_sources, const gp_p
 		if (opts) o = *opts; else gp_ptp_opts_default(&o);
 		const gp::Che &m = mesh->m;
 		// The BFS order the caller asked for (the reference's sorted_index)
-		// is built on a host thread while the solve runs.
+		// is worked out while the solve runs: on the device where the plan is
+		// built there, else on a host thread (a 1M-vertex mesh: 2.2 ms of one
+		// compute unit beside the sweeps, ~30 ms on the host, which is longer
+		// than the whole solve).
 		int rc0 = GP_OK;
 		std::string err0;
 		std::thread bfs;
-		if (sorted_out) {
+		const bool dev_order = sorted_out && gp::plan_order_possible(m, o);
+		if (sorted_out && !dev_order) {
 			bfs = std::thread([&] {
 				try {
 					std::vector<uint32_t> lev(m.nv), lim;
@@ -318,13 +322,21 @@ int gp_ptp(gp_che *mesh, const uint32_t *sources, uint32_t n_sources, const gp_p
 			~Join() { if (t.joinable()) t.join(); }
 		} join{ bfs };
 		gp_plan *p = nullptr;
-		int rc = plan_create_any(mesh, sources, n_sources, nullptr, o, &p);
+		int rc = plan_create_any(mesh, sources, n_sources, nullptr, o, &p, dev_order);
 		if (rc) return rc;
 		std::unique_ptr<gp_plan, void (*)(gp_plan *)> guard(p, gp_plan_destroy);
 		rc = gp::plan_run(p, stats);
 		if (rc) return rc;
 		rc = gp::plan_result(p, dist);
 		if (rc) return rc;
+		if (dev_order) {
+			bool have = false;
+			if ((rc = gp::plan_order(p, sorted_out, have))) return rc;
+			if (!have) {
+				std::vector<uint32_t> lev(m.nv), lim;
+				return gp::toplesets_host(m, sources, n_sources, lev.data(), sorted_out, lim);
+			}
+		}
 		if (bfs.joinable()) bfs.join();
 		if (rc0) return gp::fail(rc0, "%s", err0.c_str());
 		return GP_OK;
@@ -336,7 +348,7 @@ int gp_ptp(gp_che *mesh, const uint32_t *sources, uint32_t n_sources, const gp_p
 // Plan of any schedule: rings, or bands from dhat (caller-supplied for the
 // learned schedule; Euclidean distance or ring index otherwise).
 static int plan_create_any(gp_che *mesh, const uint32_t *sources, uint32_t n_sources, const double *dhat,
-                           const gp_ptp_opts &o, gp_plan **out)
+                           const gp_ptp_opts &o, gp_plan **out, bool want_order)
 {
 	const gp::Che &m = mesh->m;
 	if (o.fp32_geometry != GP_GEO_AUTO && o.fp32_geometry != GP_GEO_FP32 && o.fp32_geometry != GP_GEO_FP64)
@@ -356,7 +368,7 @@ static int plan_create_any(gp_che *mesh, const uint32_t *sources, uint32_t n_sou
 	// ordinary one); those meshes take the host build, which rebuilds it too.
 	const bool dev_ok = m.manifold;
 	if (dev_ok && o.device_setup && o.schedule == GP_SCHED_RINGS && o.coalesce && !o.clusters) {
-		const int rd = gp::plan_create_device(&mesh->m, sources, n_sources, o, out);
+		const int rd = gp::plan_create_device(&mesh->m, sources, n_sources, o, out, nullptr, 0, nullptr, want_order);
 		if (rd != GP_ERR_CAPACITY) return rd;
 		gp::clear_error();   // a fan too long for the device build: build on the host
 	}

@@ -130,7 +130,8 @@ int build_che(const double *xyz, uint32_t nv, const uint32_t *faces, uint32_t nf
 	// Fans.
 	m.fan_off.assign(nv + 1, 0);
 	m.fan_closed.assign(nv, 0);
-	#pragma omp parallel for schedule(static)
+	uint32_t max_link = 0;
+	#pragma omp parallel for schedule(static) reduction(max : max_link)
 	for (int64_t v = 0; v < (int64_t) nv; v++) {
 		const uint32_t stop = m.evt[v];
 		if (stop == NIL) continue;
@@ -144,7 +145,9 @@ int build_che(const double *xyz, uint32_t nv, const uint32_t *faces, uint32_t nf
 		}
 		m.fan_off[v + 1] = c + 1;
 		m.fan_closed[v] = closed;
+		max_link = std::max(max_link, closed ? c : c + 1);
 	}
+	m.max_link = max_link;
 	for (uint32_t v = 0; v < nv; v++) m.fan_off[v + 1] += m.fan_off[v];
 	m.fan.assign(m.fan_off[nv], NIL);
 	// Mean edge length: per-vertex sums added in vertex order, so the value

@@ -37,6 +37,7 @@ struct Che {
 	std::vector<uint32_t> fan;        // fan lists
 	std::vector<uint8_t> fan_closed;  // 1 when the walk returned to EVT[v]
 	double mean_edge = 1.0;           // mean length of the fan edges
+	uint32_t max_link = 0;            // longest link
 
 	DeviceMesh *dev = nullptr;        // lazily uploaded device tables
 	// Fan triangles taking the FP64 update (the flag test of build_layout) and
@@ -176,7 +177,13 @@ int plan_create_rings(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_
 // With mlp (and no dhat), dhat is the network's prediction, computed on the
 // device from the plan's own BFS levels (gp_plan_create_learned).
 int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp_opts &opts, gp_plan **out,
-                       const double *dhat = nullptr, double width = 0, gp_mlp *mlp = nullptr);
+                       const double *dhat = nullptr, double width = 0, gp_mlp *mlp = nullptr,
+                       bool want_order = false);
+// Whether a plan of these options, made with want_order, works out the
+// reference's order (sorted) on the device, and that order (waits for it; have =
+// false: the plan has none).
+bool plan_order_possible(const Che &m, const gp_ptp_opts &o);
+int plan_order(gp_plan *p, uint32_t *sorted, bool &have);
 // BFS levels of the sources computed on the device (NIL where unreached).
 int levels_gpu(Che &m, const uint32_t *src, uint32_t ns, uint32_t *levels);
 int plan_run(gp_plan *p, gp_ptp_stats *stats);

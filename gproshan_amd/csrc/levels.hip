@@ -419,8 +419,10 @@ int Levels::create(DeviceMesh *mesh, hipStream_t s)
 	    hipMalloc(&sorted, 4ull * nv) != hipSuccess || hipMalloc(&cslots, 4ull * (nchunks() + 1)) != hipSuccess ||
 	    hipMalloc(&coff, 4ull * (nchunks() + 1)) != hipSuccess ||
 	    hipMalloc(&limits, 4ull * (nv + 2)) != hipSuccess || hipMalloc(&nl, 4) != hipSuccess ||
-	    hipMalloc(&ls, sizeof(LevelState)) != hipSuccess || hipHostMalloc(&h_ls, 2 * sizeof(LevelState)) != hipSuccess)
+	    hipMalloc(&ls, sizeof(LevelState)) != hipSuccess || hipHostMalloc(&h_ls, 3 * sizeof(LevelState)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "levels: device allocation failed");
+	static_assert(sizeof(LevelInfo) <= sizeof(LevelState), "the sizes take a third snapshot's room");
+	h_info = (LevelInfo *) (h_ls + 2);
 	GP_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
 	GP_HIP(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
 	k_lv_zero<<<fill_grid(nv), 256, 0, stream>>>(mark, nv);
@@ -482,6 +484,34 @@ void Levels::sort()
 	const uint32_t nc = nchunks();
 	k_lv_chunk_slots<<<fill_grid(64 * nc), 256, 0, stream>>>(sorted, limits, nl, dm->fan_off, dm->closed, nc, cslots);
 	k_exclusive_scan<<<1, 1024, 0, stream>>>(cslots, nc, coff);
+}
+
+// The four sizes a plan is built from, in one wait instead of a copy each.
+__global__ __launch_bounds__(1024) void k_lv_info(const uint32_t *limits, const uint32_t *nl, const uint32_t *coff,
+                                                  uint32_t max_nl, LevelInfo *out)
+{
+	__shared__ uint32_t red[16];
+	const uint32_t n = min(*nl, max_nl);
+	uint32_t m = 0;
+	for (uint32_t q = 1 + threadIdx.x; q < n; q += 1024) m = max(m, limits[q] - limits[q - 1]);
+	for (uint32_t o = 32; o > 0; o >>= 1) m = max(m, (uint32_t) __shfl_xor(m, o));
+	if ((threadIdx.x & 63u) == 0) red[threadIdx.x >> 6] = m;
+	__syncthreads();
+	if (threadIdx.x != 0) return;
+	for (uint32_t q = 1; q < 16; q++) m = max(m, red[q]);
+	const uint32_t nr = n ? limits[n - 1] : 0u;
+	*out = LevelInfo{ *nl, nr, coff[(nr + 63) / 64], m };
+}
+
+int Levels::info(LevelInfo &out)
+{
+	k_lv_info<<<1, 1024, 0, stream>>>(limits, nl, coff, nv + 2, h_info);
+	GP_HIP(hipGetLastError());
+	GP_HIP(hipStreamSynchronize(stream));
+	out = *h_info;
+	if (out.nl < 2 || out.nl > nv + 1 || out.nr > nv)
+		return fail(GP_ERR_KERNEL, "levels: bad ring count %u", out.nl);
+	return GP_OK;
 }
 
 // BFS levels of the sources (NIL where unreached) on the device, copied into

@@ -21,6 +21,12 @@ struct LevelState;
 
 constexpr uint32_t LEVEL_KEYS = 8;   // slot classes per level in the sort key
 
+// Sizes of sorted rings: |limits|, reached vertices, their chunks' slot rows,
+// the widest ring.
+struct LevelInfo {
+	uint32_t nl, nr, rows, max_ring;
+};
+
 struct Levels {
 	uint32_t nv = 0;
 	uint32_t *level = nullptr;    // [nv], NIL = unreached
@@ -35,6 +41,7 @@ struct Levels {
 	uint32_t *cslots = nullptr;   // [nchunks() + 1] slot rows of each 64-position chunk of sorted
 	uint32_t *coff = nullptr;     // [nchunks() + 1] their exclusive prefix (chunk c at row coff[c])
 	LevelState *ls = nullptr, *h_ls = nullptr;   // h_ls: two pinned snapshots
+	LevelInfo *h_info = nullptr;  // pinned (behind the snapshots)
 	hipEvent_t ev[2] = { nullptr, nullptr };
 	hipStream_t stream = nullptr;   // borrowed
 	DeviceMesh *dm = nullptr;
@@ -48,7 +55,26 @@ struct Levels {
 	void seed(const uint32_t *d_src, uint32_t first, uint32_t ns);   // d_src[first, ns) to level 0
 	int expand();                                               // BFS to completion
 	void sort();                                                // sorted, limits, nl, coff on the device
+	int info(LevelInfo &out);                                   // sizes of the last sort (waits for it)
 	uint32_t nchunks() const { return (nv + 63) / 64; }
+};
+
+// Reference order of the sorted rings (rings.hip): ring_order_queue enqueues the
+// kernels that write sorted_out[nv] (device; NIL past the reached vertices) in
+// the discovery order of che::compute_toplesets from rings sorted as sets
+// (lv.sorted, lv.limits, lv.level and inv[nv], the position of each vertex in
+// lv.sorted; d_src: the sources in the caller's order).  Everything passed stays
+// unchanged and allocated until the stream has run them.
+constexpr uint32_t ORDER_MAX_LINK = 32;   // longer links: the one-workgroup BFS of rings.hip
+
+struct RingOrder {
+	uint32_t *child = nullptr, *rank0 = nullptr, *work = nullptr, *out = nullptr;
+	~RingOrder()
+	{
+		for (void *p : { (void *) child, (void *) rank0, (void *) work, (void *) out }) (void) hipFree(p);
+	}
+	int queue(const Levels &lv, const LevelInfo &li, const uint32_t *limits, const uint32_t *inv, const uint32_t *d_src,
+	          uint32_t ns, hipStream_t stream);
 };
 
 }  // namespace gp
