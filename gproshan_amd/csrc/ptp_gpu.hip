@@ -243,6 +243,7 @@ struct gp_plan {
 	uint32_t big = 64, small = 8;            // sweeps per graph replay (multiples of 4)
 	uint32_t xblk = 0;                       // log2 of the chunk blocks dealt to XCDs (0: eighths)
 	bool has_run = false;
+	bool ran_once = false;                   // a run has begun (the next may build graphs)
 	bool capped = false;                     // the last run stopped at its sweep cap
 	uint32_t check_sweeps = 0;               // check sweeps of the last run (band plans)
 	// Dataflow launch (GP_LAUNCH_FLOW): eligibility (-1: not yet checked) and buffers.
@@ -903,7 +904,13 @@ int plan_run(gp_plan *p, gp_ptp_stats *stats)
 		if (rc) return rc;
 	}
 	p->flow_last = flow;
-	const bool graph = !flow && p->opts.launch_mode == GP_LAUNCH_GRAPH && graphs_enabled();
+	// Graphs pay from the second FP32 run of a plan: building the two takes
+	// 0.35-1 ms, and a replayed sweep starts 0.2-0.4 us sooner than a launched one
+	// where the sweeps are short (4.7 against 5.2 us at 900-vertex windows, 6.7
+	// against 7.1 at 158k).  FP64 sweeps hide the launches: 6.7 against 6.3 us and
+	// 13.5 against 13.3 there, so they never build any.
+	const bool graph = !flow && !f64 && p->ran_once && p->opts.launch_mode == GP_LAUNCH_GRAPH && graphs_enabled();
+	p->ran_once = true;
 	if (graph && !p->g_big) {
 		int rc = capture(p, a, BIG, &p->g_big);
 		if (!rc) rc = capture(p, a, SMALL, &p->g_small);
