@@ -253,7 +253,7 @@ namespace gp {
 template <typename V>
 static int up(V *&dst, const V *src, size_t n)
 {
-	if (hipMalloc(&dst, sizeof(V) * std::max<size_t>(n, 1)) != hipSuccess) return fail(GP_ERR_NOMEM, "batch: allocation failed");
+	if (device_malloc(&dst, sizeof(V) * std::max<size_t>(n, 1)) != hipSuccess) return fail(GP_ERR_NOMEM, "batch: allocation failed");
 	if (n) GP_HIP(hipMemcpy(dst, src, sizeof(V) * n, hipMemcpyHostToDevice));
 	return GP_OK;
 }
@@ -295,11 +295,11 @@ static int batch_configure(gp_batch *b, uint32_t block)
 	const size_t cap = std::max<size_t>(1, (32ull << 30) / std::max<size_t>(per_wg, 1));
 	grid = (uint32_t) std::min<size_t>(grid, cap);
 	const size_t g = grid;
-	if (hipMalloc(&b->d_level, 4 * mv * g) != hipSuccess || hipMalloc(&b->d_sorted, 4 * mv * g) != hipSuccess ||
-	    hipMalloc(&b->d_limits, 4 * (mv + 2) * g) != hipSuccess || hipMalloc(&b->d_nlim, 4 * g) != hipSuccess ||
-	    hipMalloc(&b->d_key, 8 * mv * g) != hipSuccess || hipMalloc(&b->d_dist, 8 * mv * g) != hipSuccess ||
-	    hipMalloc(&b->d_finv, 4 * mv * g) != hipSuccess || hipMalloc(&b->d_fcid, 4 * fslots * g) != hipSuccess ||
-	    hipMalloc(&b->d_fmidx, 4 * fslots * g) != hipSuccess || hipMalloc(&b->d_fgeo, sizeof(float2) * fslots * g) != hipSuccess) {
+	if (device_malloc(&b->d_level, 4 * mv * g) != hipSuccess || device_malloc(&b->d_sorted, 4 * mv * g) != hipSuccess ||
+	    device_malloc(&b->d_limits, 4 * (mv + 2) * g) != hipSuccess || device_malloc(&b->d_nlim, 4 * g) != hipSuccess ||
+	    device_malloc(&b->d_key, 8 * mv * g) != hipSuccess || device_malloc(&b->d_dist, 8 * mv * g) != hipSuccess ||
+	    device_malloc(&b->d_finv, 4 * mv * g) != hipSuccess || device_malloc(&b->d_fcid, 4 * fslots * g) != hipSuccess ||
+	    device_malloc(&b->d_fmidx, 4 * fslots * g) != hipSuccess || device_malloc(&b->d_fgeo, sizeof(float2) * fslots * g) != hipSuccess) {
 		b->free_scratch();
 		return fail(GP_ERR_NOMEM, "batch: scratch allocation failed (%u workgroups x %u vertices)", grid, b->max_nv);
 	}
@@ -407,7 +407,7 @@ int batch_create(Che *const *meshes, uint32_t nmeshes, const uint32_t *job_mesh,
 	b->total_out = off;
 	int rc;
 	if ((rc = up(b->d_meshes, bm.data(), bm.size())) || (rc = up(b->d_jobs, jobs.data(), jobs.size()))) return rc;
-	if (hipMalloc(&b->d_queue, 4) != hipSuccess || hipMalloc(&b->d_out, 4 * std::max<size_t>(off, 1)) != hipSuccess)
+	if (device_malloc(&b->d_queue, 4) != hipSuccess || device_malloc(&b->d_out, 4 * std::max<size_t>(off, 1)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "batch: output allocation failed (%llu values)", off);
 	GP_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
 	GP_HIP(hipEventCreate(&b->e0));

@@ -6,6 +6,7 @@
 #include <cstdlib>
 
 #include "gp_internal.hpp"
+#include "pool.hpp"
 
 namespace gp {
 
@@ -28,6 +29,7 @@ struct DeviceMesh {
 	uint8_t *closed = nullptr; // 1 when the fan of v is closed (link = first m entries)
 	float h = 1.f, inv_h = 1.f;
 	MasterLayout *master[2] = { nullptr, nullptr };   // vertex-major slot tables (FP32, FP64), built on demand
+	bool counted = false;      // among the pool's meshes
 	uint32_t *link8 = nullptr; // first 8 link entries of each vertex (levels.hip), built on demand
 };
 

@@ -248,24 +248,25 @@ struct FpsRun {
 	hipGraphExec_t g_big = nullptr, g_small = nullptr;
 	~FpsRun()
 	{
+		if (stream) (void) hipStreamSynchronize(stream);
 		for (void *p : { (void *) cid, (void *) midx, (void *) inv, (void *) samples, (void *) cgeo, (void *) cx64,
 		                 d0, d1, (void *) st, (void *) job })
-			(void) hipFree(p);
-		if (h_st) (void) hipHostFree(h_st);
+			(void) pool_free(p);
+		pinned_free(h_st);
 		if (g_big) (void) hipGraphExecDestroy(g_big);
 		if (g_small) (void) hipGraphExecDestroy(g_small);
 		if (e0) (void) hipEventDestroy(e0);
 		if (e1) (void) hipEventDestroy(e1);
 		for (hipEvent_t e : ev)
 			if (e) (void) hipEventDestroy(e);
-		if (stream) (void) hipStreamDestroy(stream);
+		pool_stream_free(stream);
 	}
 };
 
 template <typename V>
 static int fup(V *&dst, const V *src, size_t n)
 {
-	if (hipMalloc(&dst, sizeof(V) * std::max<size_t>(n, 1)) != hipSuccess) return fail(GP_ERR_NOMEM, "fps: allocation failed");
+	if (pool_malloc(&dst, sizeof(V) * std::max<size_t>(n, 1)) != hipSuccess) return fail(GP_ERR_NOMEM, "fps: allocation failed");
 	if (n) GP_HIP(hipMemcpy(dst, src, sizeof(V) * n, hipMemcpyHostToDevice));
 	return GP_OK;
 }
@@ -294,17 +295,17 @@ static int fps_impl(Che &m, uint32_t *samples, uint32_t n_init, uint32_t cap, ui
 	// streaming loop.
 	const uint32_t nchunks = (nv + 63) / 64, npos = nchunks * 64;
 	const size_t lanes = (size_t) nchunks * S * 64;
-	if (hipMalloc(&r.cid, 4 * lanes) != hipSuccess || hipMalloc(&r.inv, 4ull * nv) != hipSuccess ||
-	    (F64 ? hipMalloc(&r.cx64, sizeof(Edge64) * lanes)
-	         : (hipMalloc(&r.cgeo, sizeof(float2) * lanes) == hipSuccess ? hipMalloc(&r.midx, 4 * lanes)
+	if (pool_malloc(&r.cid, 4 * lanes) != hipSuccess || pool_malloc(&r.inv, 4ull * nv) != hipSuccess ||
+	    (F64 ? pool_malloc(&r.cx64, sizeof(Edge64) * lanes)
+	         : (pool_malloc(&r.cgeo, sizeof(float2) * lanes) == hipSuccess ? pool_malloc(&r.midx, 4 * lanes)
 	                                                                      : hipErrorOutOfMemory)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "fps: table allocation failed");
 	if ((rc = fup(r.samples, samples, cap))) return rc;
-	if (hipMalloc(&r.d0, sizeof(T) * nv) != hipSuccess || hipMalloc(&r.d1, sizeof(T) * nv) != hipSuccess ||
-	    hipMalloc(&r.st, sizeof(FState)) != hipSuccess || hipMalloc(&r.job, sizeof(BfsJob)) != hipSuccess ||
-	    hipHostMalloc(&r.h_st, 3 * sizeof(FState)) != hipSuccess)
+	if (pool_malloc(&r.d0, sizeof(T) * nv) != hipSuccess || pool_malloc(&r.d1, sizeof(T) * nv) != hipSuccess ||
+	    pool_malloc(&r.st, sizeof(FState)) != hipSuccess || pool_malloc(&r.job, sizeof(BfsJob)) != hipSuccess ||
+	    pinned_malloc(&r.h_st, 3 * sizeof(FState)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "fps: device allocation failed");
-	GP_HIP(hipStreamCreateWithFlags(&r.stream, hipStreamNonBlocking));
+	GP_HIP(pool_stream(&r.stream));
 	Levels lv;
 	if ((rc = lv.create(m.dev, r.stream))) return rc;
 	const BfsJob job{ r.samples, n_init, lv.level, nullptr, lv.sorted, lv.limits, lv.nl };

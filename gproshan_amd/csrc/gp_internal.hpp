@@ -215,6 +215,9 @@ void patch_destroy(PatchPlan *pp);
 const char *last_error();
 void clear_error();
 
+// memcpy by several threads when it is large (copy_out.cpp).
+void copy_out(void *dst, const void *src, size_t bytes);
+
 // Learned band predictor (mlp.hip).
 constexpr uint32_t MLP_NPARAM = 64 * 32 + 64 + 64 * 64 + 64 + 64 + 1;
 int fps_gpu(Che &m, uint32_t *samples, uint32_t n_init, uint32_t cap, uint64_t n, double radio, bool f64,

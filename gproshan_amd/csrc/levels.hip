@@ -378,10 +378,11 @@ __global__ __launch_bounds__(1024) void k_exclusive_scan(const uint32_t *in, uin
 
 Levels::~Levels()
 {
+	if (stream) (void) hipStreamSynchronize(stream);
 	for (void *p : { (void *) level, (void *) queue, (void *) mark, (void *) hist, (void *) sorted, (void *) limits,
 	                 (void *) nl, (void *) ls, (void *) cslots, (void *) coff })
-		(void) hipFree(p);
-	if (h_ls) (void) hipHostFree(h_ls);
+		(void) pool_free(p);
+	pinned_free(h_ls);
 	for (hipEvent_t e : ev)
 		if (e) (void) hipEventDestroy(e);
 }
@@ -395,7 +396,7 @@ static int link_rows(DeviceMesh *dm)
 	std::lock_guard<std::mutex> lock(mu);
 	if (dm->link8) return GP_OK;
 	uint32_t *p = nullptr;
-	if (hipMalloc(&p, 4ull * LINK_ROW * dm->nv) != hipSuccess)
+	if (device_malloc(&p, 4ull * LINK_ROW * dm->nv) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "levels: device allocation failed");
 	k_link8<<<fill_grid(dm->nv), 256>>>(dm->fan_off, dm->fan, dm->closed, dm->nv, p);
 	const hipError_t e = hipGetLastError() != hipSuccess ? hipErrorUnknown : hipDeviceSynchronize();
@@ -413,13 +414,13 @@ int Levels::create(DeviceMesh *mesh, hipStream_t s)
 	nv = mesh->nv;
 	stream = s;
 	if (int rc = link_rows(mesh)) return rc;
-	if (hipMalloc(&level, 4ull * nv) != hipSuccess || hipMalloc(&queue, 8ull * nv) != hipSuccess ||
-	    hipMalloc(&mark, 4ull * nv) != hipSuccess ||
-	    hipMalloc(&hist, 4ull * ((size_t) nv * LEVEL_KEYS + 1)) != hipSuccess ||
-	    hipMalloc(&sorted, 4ull * nv) != hipSuccess || hipMalloc(&cslots, 4ull * (nchunks() + 1)) != hipSuccess ||
-	    hipMalloc(&coff, 4ull * (nchunks() + 1)) != hipSuccess ||
-	    hipMalloc(&limits, 4ull * (nv + 2)) != hipSuccess || hipMalloc(&nl, 4) != hipSuccess ||
-	    hipMalloc(&ls, sizeof(LevelState)) != hipSuccess || hipHostMalloc(&h_ls, 3 * sizeof(LevelState)) != hipSuccess)
+	if (pool_malloc(&level, 4ull * nv) != hipSuccess || pool_malloc(&queue, 8ull * nv) != hipSuccess ||
+	    pool_malloc(&mark, 4ull * nv) != hipSuccess ||
+	    pool_malloc(&hist, 4ull * ((size_t) nv * LEVEL_KEYS + 1)) != hipSuccess ||
+	    pool_malloc(&sorted, 4ull * nv) != hipSuccess || pool_malloc(&cslots, 4ull * (nchunks() + 1)) != hipSuccess ||
+	    pool_malloc(&coff, 4ull * (nchunks() + 1)) != hipSuccess ||
+	    pool_malloc(&limits, 4ull * (nv + 2)) != hipSuccess || pool_malloc(&nl, 4) != hipSuccess ||
+	    pool_malloc(&ls, sizeof(LevelState)) != hipSuccess || pinned_malloc(&h_ls, 3 * sizeof(LevelState)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "levels: device allocation failed");
 	static_assert(sizeof(LevelInfo) <= sizeof(LevelState), "the sizes take a third snapshot's room");
 	h_info = (LevelInfo *) (h_ls + 2);
@@ -523,12 +524,12 @@ int levels_gpu(Che &m, const uint32_t *src, uint32_t ns, uint32_t *levels)
 		if (src[q] >= m.nv) return fail(GP_ERR_INVALID, "levels: source %u out of range", src[q]);
 	int rc = upload_mesh(m);
 	if (rc) return rc;
-	hipStream_t stream = nullptr;
-	GP_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-	std::unique_ptr<std::remove_pointer<hipStream_t>::type, hipError_t (*)(hipStream_t)> sg(stream, hipStreamDestroy);
-	uint32_t *d_src = nullptr;
-	if (hipMalloc(&d_src, 4ull * ns) != hipSuccess) return fail(GP_ERR_NOMEM, "levels: device allocation failed");
-	std::unique_ptr<uint32_t, hipError_t (*)(void *)> dg(d_src, hipFree);
+	PoolStream ps;
+	GP_HIP(ps.create());
+	const hipStream_t stream = ps.s;
+	PoolBuf<uint32_t> srcb(stream);
+	if (srcb.alloc(4ull * ns) != hipSuccess) return fail(GP_ERR_NOMEM, "levels: device allocation failed");
+	uint32_t *const d_src = srcb.p;
 	GP_HIP(hipMemcpy(d_src, src, 4ull * ns, hipMemcpyHostToDevice));
 	Levels lv;
 	if ((rc = lv.create(m.dev, stream))) return rc;

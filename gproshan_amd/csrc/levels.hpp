@@ -69,12 +69,14 @@ constexpr uint32_t ORDER_MAX_LINK = 32;   // longer links: the one-workgroup BFS
 
 struct RingOrder {
 	uint32_t *child = nullptr, *rank0 = nullptr, *work = nullptr, *out = nullptr;
+	hipStream_t stream = nullptr;   // the one it was queued on
 	~RingOrder()
 	{
-		for (void *p : { (void *) child, (void *) rank0, (void *) work, (void *) out }) (void) hipFree(p);
+		if (stream) (void) hipStreamSynchronize(stream);
+		for (void *p : { (void *) child, (void *) rank0, (void *) work, (void *) out }) (void) pool_free(p);
 	}
 	int queue(const Levels &lv, const LevelInfo &li, const uint32_t *limits, const uint32_t *inv, const uint32_t *d_src,
-	          uint32_t ns, hipStream_t stream);
+	          uint32_t ns, hipStream_t on);
 };
 
 }  // namespace gp

@@ -517,9 +517,9 @@ int mlp_create(uint32_t seed, gp_mlp **out)
 	int rc = device_check(nullptr, 0);
 	if (rc) return rc;
 	auto m = std::make_unique<gp_mlp>();
-	if (hipMalloc(&m->d.w, 4 * NPARAM) != hipSuccess || hipMalloc(&m->d.m, 4 * NPARAM) != hipSuccess ||
-	    hipMalloc(&m->d.v, 4 * NPARAM) != hipSuccess || hipMalloc(&m->d.w1, 2 * HD * KP) != hipSuccess ||
-	    hipMalloc(&m->d.w2, 2 * HD * HD) != hipSuccess || hipMalloc(&m->d.w2t, 2 * HD * HD) != hipSuccess)
+	if (device_malloc(&m->d.w, 4 * NPARAM) != hipSuccess || device_malloc(&m->d.m, 4 * NPARAM) != hipSuccess ||
+	    device_malloc(&m->d.v, 4 * NPARAM) != hipSuccess || device_malloc(&m->d.w1, 2 * HD * KP) != hipSuccess ||
+	    device_malloc(&m->d.w2, 2 * HD * HD) != hipSuccess || device_malloc(&m->d.w2t, 2 * HD * HD) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "mlp: allocation failed");
 	// He initialisation (normal), zero biases, zero padding columns.
 	std::vector<float> w(NPARAM, 0.f);
@@ -552,10 +552,19 @@ int mlp_params(gp_mlp *m, float *get, const float *set, uint32_t n)
 
 struct DevBuf {
 	void *p = nullptr;
-	~DevBuf() { if (p) (void) hipFree(p); }
+	hipStream_t s = nullptr;   // the stream that uses it
+	DevBuf(hipStream_t stream = nullptr) : s(stream) {}
+	DevBuf(const DevBuf &) = delete;
+	DevBuf &operator=(const DevBuf &) = delete;
+	~DevBuf()
+	{
+		if (!p) return;
+		(void) hipStreamSynchronize(s);
+		(void) pool_free(p);
+	}
 	int alloc(size_t b)
 	{
-		if (hipMalloc(&p, std::max<size_t>(b, 4)) != hipSuccess) return fail(GP_ERR_NOMEM, "device allocation failed");
+		if (pool_malloc(&p, std::max<size_t>(b, 4)) != hipSuccess) return fail(GP_ERR_NOMEM, "device allocation failed");
 		return GP_OK;
 	}
 };
@@ -656,7 +665,7 @@ int mlp_predict_device(gp_mlp *m, Che &mesh, const uint32_t *d_src, uint32_t ns,
 	const hipStream_t stream = (hipStream_t) stream_;
 	int rc = upload_mesh(mesh);
 	if (rc) return rc;
-	DevBuf X, e, y;
+	DevBuf X(stream), e(stream), y(stream);
 	const uint32_t nv = mesh.nv;
 	if ((rc = X.alloc(2ull * KP * nv)) || (rc = e.alloc(4ull * nv)) || (rc = y.alloc(4ull * nv))) return rc;
 	FeatArgs a{ mesh.dev->fan_off, mesh.dev->fan, mesh.dev->closed, mesh.dev->pos, d_src, ns, d_levels, lmax, nv,

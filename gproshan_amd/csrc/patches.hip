@@ -371,7 +371,7 @@ struct PatchPlan {
 template <typename V>
 static int pupload(V *&dst, const V *src, size_t n)
 {
-	if (hipMalloc(&dst, sizeof(V) * std::max<size_t>(n, 1)) != hipSuccess) return fail(GP_ERR_NOMEM, "patch plan: allocation failed");
+	if (device_malloc(&dst, sizeof(V) * std::max<size_t>(n, 1)) != hipSuccess) return fail(GP_ERR_NOMEM, "patch plan: allocation failed");
 	if (n) GP_HIP(hipMemcpy(dst, src, sizeof(V) * n, hipMemcpyHostToDevice));
 	return GP_OK;
 }
@@ -451,10 +451,10 @@ int patch_create(Che *mesh, const uint32_t *src, uint32_t ns, const double *dhat
 	    (rc = pupload(pp->d_src, srcm.data(), srcm.size())))
 		return rc;
 	const uint32_t trace_rows = std::min<uint32_t>(pp->max_launch, 1u << 20);
-	if (hipMalloc(&pp->d_list, 4ull * 4 * pp->npatch) != hipSuccess ||
-	    hipMalloc(&pp->d_mark, 4ull * 4 * pp->npatch) != hipSuccess || hipMalloc(&pp->d_defer, pp->npatch) != hipSuccess ||
-	    hipMalloc(&pp->d_trace, 32ull * trace_rows) != hipSuccess || hipMalloc(&pp->d_dist, 4ull * pp->n) != hipSuccess ||
-	    hipMalloc(&pp->d_out, 8ull * pp->n) != hipSuccess || hipMalloc(&pp->d_state, sizeof(PatchState)) != hipSuccess ||
+	if (device_malloc(&pp->d_list, 4ull * 4 * pp->npatch) != hipSuccess ||
+	    device_malloc(&pp->d_mark, 4ull * 4 * pp->npatch) != hipSuccess || device_malloc(&pp->d_defer, pp->npatch) != hipSuccess ||
+	    device_malloc(&pp->d_trace, 32ull * trace_rows) != hipSuccess || device_malloc(&pp->d_dist, 4ull * pp->n) != hipSuccess ||
+	    device_malloc(&pp->d_out, 8ull * pp->n) != hipSuccess || device_malloc(&pp->d_state, sizeof(PatchState)) != hipSuccess ||
 	    hipHostMalloc(&pp->h_state, sizeof(PatchState)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "patch plan: device allocation failed");
 	pp->max_launch = std::min(pp->max_launch, trace_rows);

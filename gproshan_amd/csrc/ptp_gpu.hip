@@ -60,7 +60,9 @@ void device_mesh_free(DeviceMesh *d)
 	delete d->master[0];
 	delete d->master[1];
 	(void) hipFree(d->link8);
+	const bool counted = d->counted;
 	delete d;
+	if (counted) pool_mesh_removed();
 }
 
 int device_check(char *name, size_t cap)
@@ -96,16 +98,18 @@ int upload_mesh(Che &m)
 	dm->nv = nv; dm->nfan = nfan;
 	dm->h = (float) m.mean_edge; dm->inv_h = (float) (1.0 / m.mean_edge);
 	auto cleanup = [&](int r) { device_mesh_free(dm.release()); return r; };
-	if (hipMalloc(&dm->fan_off, sizeof(uint32_t) * (nv + 1)) != hipSuccess ||
-	    hipMalloc(&dm->fan, sizeof(uint32_t) * std::max<uint32_t>(nfan, 1)) != hipSuccess ||
-	    hipMalloc(&dm->pos, sizeof(double) * 3 * (size_t) nv) != hipSuccess ||
-	    hipMalloc(&dm->closed, nv) != hipSuccess)
+	if (device_malloc(&dm->fan_off, sizeof(uint32_t) * (nv + 1)) != hipSuccess ||
+	    device_malloc(&dm->fan, sizeof(uint32_t) * std::max<uint32_t>(nfan, 1)) != hipSuccess ||
+	    device_malloc(&dm->pos, sizeof(double) * 3 * (size_t) nv) != hipSuccess ||
+	    device_malloc(&dm->closed, nv) != hipSuccess)
 		return cleanup(fail(GP_ERR_NOMEM, "device mesh allocation failed"));
 	if (hipMemcpy(dm->fan_off, m.fan_off.data(), sizeof(uint32_t) * (nv + 1), hipMemcpyHostToDevice) != hipSuccess ||
 	    (nfan && hipMemcpy(dm->fan, m.fan.data(), sizeof(uint32_t) * nfan, hipMemcpyHostToDevice) != hipSuccess) ||
 	    hipMemcpy(dm->pos, m.gt.data(), sizeof(double) * 3 * (size_t) nv, hipMemcpyHostToDevice) != hipSuccess ||
 	    hipMemcpy(dm->closed, m.fan_closed.data(), nv, hipMemcpyHostToDevice) != hipSuccess)
 		return cleanup(fail(GP_ERR_HIP, "device mesh upload failed"));
+	dm->counted = true;
+	pool_mesh_added();
 	m.dev = dm.release();
 	return GP_OK;
 }
@@ -122,18 +126,16 @@ __global__ void k_cl_sources(uint32_t *c0, uint32_t *c1, const uint32_t *src, ui
 	if (t < ns) c0[src[t]] = c1[src[t]] = t + 1;
 }
 
-template <typename T>
-__global__ void k_to_f64(const T *in, double *out, uint32_t n)
+// Values of vertices [v0, v0 + n) from the ring positions (inv; null: the buffer
+// is in the caller's numbering), `none` where unreached, straight into pinned
+// host memory.
+template <typename T, typename O>
+__global__ void k_result(const T *in, const uint32_t *inv, uint32_t v0, uint32_t n, O none, O *out)
 {
-	const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-	for (uint32_t v = t; v < n; v += gridDim.x * blockDim.x) out[v] = (double) in[v];
-}
-
-// Device-built plans: the result in the caller's numbering.
-__global__ void k_from_positions(const double *in, const uint32_t *inv, uint32_t nv, double *out)
-{
-	for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < nv; v += gridDim.x * blockDim.x)
-		out[v] = inv[v] != GP_NIL ? in[inv[v]] : (double) INFINITY;
+	for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
+		const uint32_t p = inv ? inv[v0 + q] : v0 + q;
+		out[q] = p != GP_NIL ? (O) in[p] : none;
+	}
 }
 
 __global__ void k_fill_u32(uint32_t *p, uint32_t n, uint32_t x)
@@ -233,9 +235,7 @@ struct gp_plan {
 	gp::Edge64 *d_cx64 = nullptr;
 	void *d_dist0 = nullptr, *d_dist1 = nullptr;
 	uint32_t *d_cl0 = nullptr, *d_cl1 = nullptr;   // cluster labels (opts.clusters)
-	uint32_t *d_inv = nullptr;                // device-built plans: original vertex -> position (NIL: unreached)
-	double *d_out = nullptr;
-	double *d_orig = nullptr;                 // device-built plans: the result in the original numbering
+	uint32_t *d_inv = nullptr;                // ring-numbered plans: original vertex -> position (NIL: unreached)
 	gp::PState *d_state = nullptr, *h_state = nullptr;   // h_state: 2 pinned snapshots
 	hipStream_t stream = nullptr;
 	hipEvent_t e0 = nullptr, e1 = nullptr, ev[2] = { nullptr, nullptr };
@@ -256,29 +256,28 @@ struct gp_plan {
 
 	~gp_plan()
 	{
-		if (ostream) {
-			(void) hipStreamSynchronize(ostream);
-			(void) hipStreamDestroy(ostream);
-		}
-		(void) hipFree(d_srcv);
+		// The buffers go back to the pool: nothing may still use them.
+		if (ostream) (void) hipStreamSynchronize(ostream);
+		if (stream) (void) hipStreamSynchronize(stream);
+		lv.reset();
 		for (void *q : { (void *) d_pr0, (void *) d_pr1, (void *) d_facc, (void *) d_cflag, (void *) d_hist,
-		                 (void *) d_fs })
-			(void) hipFree(q);
-		if (h_fs) (void) hipHostFree(h_fs);
-		for (void *p : { (void *) d_limits, (void *) d_order, (void *) d_src, (void *) d_trace, (void *) d_coff,
-		                 (void *) d_cid, (void *) d_cgeo, (void *) d_cgeo64, (void *) d_cx64, d_dist0, d_dist1,
-		                 (void *) d_out, (void *) d_state, (void *) d_fcum, (void *) d_cl0, (void *) d_cl1,
-		                 (void *) d_inv, (void *) d_orig })
-			(void) hipFree(p);
+		                 (void *) d_fs, (void *) d_srcv, (void *) d_limits, (void *) d_order, (void *) d_src,
+		                 (void *) d_trace, (void *) d_coff, (void *) d_cid, (void *) d_cgeo, (void *) d_cgeo64,
+		                 (void *) d_cx64, d_dist0, d_dist1, (void *) d_state, (void *) d_fcum, (void *) d_cl0,
+		                 (void *) d_cl1, (void *) d_inv })
+			(void) gp::pool_free(q);
+		gp::pinned_free(h_fs);
 		if (pp) gp::patch_destroy(pp);
 		if (g_big) (void) hipGraphExecDestroy(g_big);
 		if (g_small) (void) hipGraphExecDestroy(g_small);
-		if (h_state) (void) hipHostFree(h_state);
+		gp::pinned_free(h_state);
 		if (e0) (void) hipEventDestroy(e0);
 		if (e1) (void) hipEventDestroy(e1);
 		for (hipEvent_t e : ev)
 			if (e) (void) hipEventDestroy(e);
-		if (stream) (void) hipStreamDestroy(stream);
+		order.stream = nullptr;              // waited for above; its stream is given back here
+		gp::pool_stream_free(ostream);
+		gp::pool_stream_free(stream);
 	}
 };
 
@@ -288,7 +287,7 @@ template <typename V>
 static int upload(V *&dst, const std::vector<typename std::remove_const<V>::type> &src)
 {
 	const size_t bytes = sizeof(V) * std::max<size_t>(src.size(), 1);
-	if (hipMalloc(&dst, bytes) != hipSuccess) return fail(GP_ERR_NOMEM, "device allocation of %zu bytes failed", bytes);
+	if (pool_malloc(&dst, bytes) != hipSuccess) return fail(GP_ERR_NOMEM, "device allocation of %zu bytes failed", bytes);
 	if (!src.empty()) GP_HIP(hipMemcpy(dst, src.data(), sizeof(V) * src.size(), hipMemcpyHostToDevice));
 	return GP_OK;
 }
@@ -317,7 +316,7 @@ static int sweep_grid(gp_plan *p, bool f64)
 
 static int plan_stream(gp_plan *p)
 {
-	GP_HIP(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking));
+	GP_HIP(pool_stream(&p->stream));
 	GP_HIP(hipEventCreate(&p->e0));
 	GP_HIP(hipEventCreate(&p->e1));
 	GP_HIP(hipEventCreate(&p->ev[0]));
@@ -330,13 +329,12 @@ static int plan_run_buffers(gp_plan *p, bool f64)
 {
 	const size_t es = f64 ? sizeof(double) : sizeof(float);
 	if (p->opts.clusters &&
-	    (hipMalloc(&p->d_cl0, 4ull * p->n) != hipSuccess || hipMalloc(&p->d_cl1, 4ull * p->n) != hipSuccess))
+	    (pool_malloc(&p->d_cl0, 4ull * p->n) != hipSuccess || pool_malloc(&p->d_cl1, 4ull * p->n) != hipSuccess))
 		return fail(GP_ERR_NOMEM, "plan: cluster allocation failed");
-	if (hipMalloc(&p->d_dist0, es * p->n) != hipSuccess || hipMalloc(&p->d_dist1, es * p->n) != hipSuccess ||
-	    hipMalloc(&p->d_out, sizeof(double) * p->n) != hipSuccess ||
-	    hipMalloc(&p->d_state, sizeof(PState)) != hipSuccess ||
-	    hipMalloc(&p->d_trace, sizeof(uint32_t) * 8 * (size_t) (p->max_iter + 1)) != hipSuccess ||
-	    hipHostMalloc(&p->h_state, 2 * sizeof(PState)) != hipSuccess)
+	if (pool_malloc(&p->d_dist0, es * p->n) != hipSuccess || pool_malloc(&p->d_dist1, es * p->n) != hipSuccess ||
+	    pool_malloc(&p->d_state, sizeof(PState)) != hipSuccess ||
+	    pool_malloc(&p->d_trace, sizeof(uint32_t) * 8 * (size_t) (p->max_iter + 1)) != hipSuccess ||
+	    pinned_malloc(&p->h_state, 2 * sizeof(PState)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "plan: device allocation failed");
 	return GP_OK;
 }
@@ -452,6 +450,7 @@ int plan_create_rings(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_
 		    (rc = upload(p->d_fcum, L.fcum)))
 			return rc;
 	}
+	if (opts.coalesce && (rc = upload(p->d_inv, p->inv))) return rc;
 	if (!opts.coalesce) {
 		std::vector<uint32_t> ord(sorted, sorted + nr);
 		if ((rc = upload(p->d_order, ord))) return rc;
@@ -535,9 +534,9 @@ int master_tables(Che &mesh, bool f64, VertexTables &out, uint32_t &max_slots)
 			m->max_slots = std::max(m->max_slots, (n && mesh.fan_closed[v]) ? n - 1 : n);
 		}
 		const size_t nf = std::max<size_t>(dm->nfan, 1);
-		if (hipMalloc(&m->cid, 4 * nf) != hipSuccess ||
-		    (f64 ? hipMalloc(&m->cx64, sizeof(Edge64) * nf)
-		         : (hipMalloc(&m->cgeo, sizeof(float2) * nf) == hipSuccess ? hipMalloc(&m->cgeo64, sizeof(double4) * nf)
+		if (device_malloc(&m->cid, 4 * nf) != hipSuccess ||
+		    (f64 ? device_malloc(&m->cx64, sizeof(Edge64) * nf)
+		         : (device_malloc(&m->cgeo, sizeof(float2) * nf) == hipSuccess ? device_malloc(&m->cgeo64, sizeof(double4) * nf)
 		                                                                  : hipErrorOutOfMemory)) != hipSuccess)
 			return fail(GP_ERR_NOMEM, "layout: device allocation failed");
 		const double ih = 1.0 / mesh.mean_edge, ih2 = ih * ih;
@@ -626,17 +625,13 @@ int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp
 		// the caller's dhat, or the network's prediction from these levels
 		// (the features' ring index), kept on the device.
 		if (!(width > 0)) return fail(GP_ERR_INVALID, "band width must be positive");
-		double *d_dhat = nullptr;
-		uint32_t *d_bmax = nullptr;
-		if (dhat) {
-			std::vector<double> dh(dhat, dhat + mesh->nv);
-			if ((rc = upload(d_dhat, dh))) return rc;
-		} else if (hipMalloc(&d_dhat, sizeof(double) * mesh->nv) != hipSuccess) {
+		PoolBuf<double> dhatb(p->stream);
+		PoolBuf<uint32_t> bmaxb(p->stream);
+		if (dhatb.alloc(sizeof(double) * mesh->nv) != hipSuccess || bmaxb.alloc(4) != hipSuccess)
 			return fail(GP_ERR_NOMEM, "plan: device allocation failed");
-		}
-		std::unique_ptr<double, hipError_t (*)(void *)> dhat_guard(d_dhat, hipFree);
-		if (hipMalloc(&d_bmax, 4) != hipSuccess) return fail(GP_ERR_NOMEM, "plan: device allocation failed");
-		std::unique_ptr<uint32_t, hipError_t (*)(void *)> bmax_guard(d_bmax, hipFree);
+		double *const d_dhat = dhatb.p;
+		uint32_t *const d_bmax = bmaxb.p;
+		if (dhat) GP_HIP(hipMemcpy(d_dhat, dhat, sizeof(double) * mesh->nv, hipMemcpyHostToDevice));
 		const uint32_t gb = std::max<uint32_t>(1, std::min<uint32_t>(2048, (mesh->nv + 255) / 256));
 		if (!dhat) {
 			k_fill_u32<<<1, 64, 0, p->stream>>>(d_bmax, 1, 0);
@@ -674,17 +669,16 @@ int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp
 	p->g64 = !f64 && opts.fp32_geometry == GP_GEO_FP64;
 	if (rows > p->nchunks * S) return fail(GP_ERR_KERNEL, "plan: bad chunk slot rows %u", rows);
 	const size_t lanes = (size_t) rows * 64;
-	if (hipMalloc(&p->d_limits, 4ull * nl) != hipSuccess || hipMalloc(&p->d_src, 4ull * ns) != hipSuccess ||
-	    hipMalloc(&p->d_inv, 4ull * mesh->nv) != hipSuccess ||
-	    hipMalloc(&p->d_orig, sizeof(double) * mesh->nv) != hipSuccess ||
-	    hipMalloc(&p->d_coff, 4ull * (p->nchunks + 1)) != hipSuccess ||
-	    hipMalloc(&p->d_cid, 4 * std::max<size_t>(lanes, 1)) != hipSuccess)
+	if (pool_malloc(&p->d_limits, 4ull * nl) != hipSuccess || pool_malloc(&p->d_src, 4ull * ns) != hipSuccess ||
+	    pool_malloc(&p->d_inv, 4ull * mesh->nv) != hipSuccess ||
+	    pool_malloc(&p->d_coff, 4ull * (p->nchunks + 1)) != hipSuccess ||
+	    pool_malloc(&p->d_cid, 4 * std::max<size_t>(lanes, 1)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "plan: device allocation failed");
 	if (f64) {
-		if (hipMalloc(&p->d_cx64, sizeof(Edge64) * std::max<size_t>(lanes, 1)) != hipSuccess)
+		if (pool_malloc(&p->d_cx64, sizeof(Edge64) * std::max<size_t>(lanes, 1)) != hipSuccess)
 			return fail(GP_ERR_NOMEM, "plan: device allocation failed");
-	} else if (hipMalloc(&p->d_cgeo, sizeof(float2) * std::max<size_t>(lanes, 1)) != hipSuccess ||
-	           hipMalloc(&p->d_cgeo64, sizeof(double4) * std::max<size_t>(lanes, 1)) != hipSuccess) {
+	} else if (pool_malloc(&p->d_cgeo, sizeof(float2) * std::max<size_t>(lanes, 1)) != hipSuccess ||
+	           pool_malloc(&p->d_cgeo64, sizeof(double4) * std::max<size_t>(lanes, 1)) != hipSuccess) {
 		return fail(GP_ERR_NOMEM, "plan: device allocation failed");
 	}
 	GP_HIP(hipMemcpyAsync(p->d_limits, lv.limits, 4ull * nl, hipMemcpyDeviceToDevice, p->stream));
@@ -704,7 +698,7 @@ int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp
 	GP_HIP(hipGetLastError());
 	GP_HIP(hipStreamSynchronize(p->stream));
 	if (want_order && opts.schedule == GP_SCHED_RINGS && mesh->max_link <= ORDER_MAX_LINK) {
-		GP_HIP(hipStreamCreateWithFlags(&p->ostream, hipStreamNonBlocking));
+		GP_HIP(pool_stream(&p->ostream));
 		if ((rc = p->order.queue(lv, li, p->d_limits, p->d_inv, d_srcv, ns, p->ostream))) return rc;
 	} else {
 		p->lv.reset();
@@ -712,6 +706,53 @@ int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp
 	if ((rc = sweep_grid(p.get(), f64))) return rc;
 	if ((rc = plan_run_buffers(p.get(), f64))) return rc;
 	*out = p.release();
+	return GP_OK;
+}
+
+// n values in the caller's numbering into host memory: written by the device to
+// pinned memory in pieces, each copied out by several threads while the next
+// are written.  A 1M-vertex field into a fresh array: 2.7 ms with a conversion
+// kernel and a pageable copy, 0.39 ms so (0.22 into pages already touched).
+template <typename T, typename O>
+static int result_out(hipStream_t stream, const T *buf, const uint32_t *inv, uint32_t n, O none, O *out)
+{
+	constexpr uint32_t PIECE = 1u << 18, ROUND = 8;   // values of a piece, pieces in flight
+	O *stage = nullptr;
+	const size_t staged = std::min<size_t>(n, (size_t) PIECE * ROUND);
+	if (pinned_malloc(&stage, sizeof(O) * staged) != hipSuccess) return fail(GP_ERR_NOMEM, "result: pinned allocation failed");
+	hipEvent_t ev[ROUND] = {};
+	struct Back {
+		O *s;
+		hipEvent_t (&ev)[ROUND];
+		hipStream_t stream;
+		~Back()
+		{
+			(void) hipStreamSynchronize(stream);
+			pinned_free(s);
+			for (hipEvent_t e : ev)
+				if (e) (void) hipEventDestroy(e);
+		}
+	} back{ stage, ev, stream };
+	for (uint32_t r0 = 0; r0 < n; r0 += PIECE * ROUND) {
+		const uint32_t rn = std::min(n - r0, PIECE * ROUND), np = (rn + PIECE - 1) / PIECE;
+		for (uint32_t q = 0; q < np; q++) {
+			const uint32_t at = q * PIECE, m = std::min(rn - at, PIECE);
+			k_result<<<std::min<uint32_t>(256, (m + 255) / 256), 256, 0, stream>>>(buf, inv, r0 + at, m, none, stage + at);
+			GP_HIP(hipGetLastError());
+			if (n <= PIECE) {
+				GP_HIP(hipStreamSynchronize(stream));
+				copy_out(out, stage, sizeof(O) * n);
+				return GP_OK;
+			}
+			if (!ev[q]) GP_HIP(hipEventCreateWithFlags(&ev[q], hipEventDisableTiming));
+			GP_HIP(hipEventRecord(ev[q], stream));
+		}
+		for (uint32_t q = 0; q < np; q++) {
+			const uint32_t at = q * PIECE, m = std::min(rn - at, PIECE);
+			GP_HIP(hipEventSynchronize(ev[q]));
+			copy_out(out + r0 + at, stage + at, sizeof(O) * m);
+		}
+	}
 	return GP_OK;
 }
 
@@ -731,9 +772,7 @@ int plan_order(gp_plan *p, uint32_t *sorted, bool &have)
 {
 	have = p && p->ostream;
 	if (!have) return GP_OK;
-	GP_HIP(hipMemcpyAsync(sorted, p->order.out, 4ull * p->nv_orig, hipMemcpyDeviceToHost, p->ostream));
-	GP_HIP(hipStreamSynchronize(p->ostream));
-	return GP_OK;
+	return result_out<uint32_t, uint32_t>(p->ostream, p->order.out, nullptr, p->nv_orig, GP_NIL, sorted);
 }
 
 static KArgs make_args(const gp_plan *p)
@@ -839,10 +878,10 @@ static int flow_prepare(gp_plan *p, bool &ok)
 	if (waves == 0 || nch > FLOW_MAX_OWN * (size_t) waves) return GP_OK;
 	p->flow_grid = waves;
 	const size_t nh = (size_t) p->max_iter + 2;
-	if (hipMalloc(&p->d_pr0, 8ull * nch * 64) != hipSuccess || hipMalloc(&p->d_pr1, 8ull * nch * 64) != hipSuccess ||
-	    hipMalloc(&p->d_facc, 8 * nh) != hipSuccess || hipMalloc(&p->d_cflag, 4ull * nch) != hipSuccess ||
-	    hipMalloc(&p->d_hist, 4 * nh) != hipSuccess || hipMalloc(&p->d_fs, sizeof(FlowState)) != hipSuccess ||
-	    hipHostMalloc(&p->h_fs, sizeof(FlowState)) != hipSuccess)
+	if (pool_malloc(&p->d_pr0, 8ull * nch * 64) != hipSuccess || pool_malloc(&p->d_pr1, 8ull * nch * 64) != hipSuccess ||
+	    pool_malloc(&p->d_facc, 8 * nh) != hipSuccess || pool_malloc(&p->d_cflag, 4ull * nch) != hipSuccess ||
+	    pool_malloc(&p->d_hist, 4 * nh) != hipSuccess || pool_malloc(&p->d_fs, sizeof(FlowState)) != hipSuccess ||
+	    pinned_malloc(&p->h_fs, sizeof(FlowState)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "plan: dataflow buffer allocation failed");
 	p->flow_ok = 1;
 	ok = true;
@@ -1049,28 +1088,9 @@ int plan_result(gp_plan *p, double *dist)
 	const uint32_t d = p->h_state->final_d;
 	const bool last_read = p->opts.result_buffer == GP_RESULT_LAST_READ;
 	const void *buf = (last_read ? !d : d) ? p->d_dist1 : p->d_dist0;
-	const uint32_t g = std::max<uint32_t>(1, std::min<uint32_t>(1024, (p->n + 255) / 256));
 	if (p->opts.precision == GP_PREC_F64)
-		k_to_f64<double><<<g, 256, 0, p->stream>>>((const double *) buf, p->d_out, p->n);
-	else
-		k_to_f64<float><<<g, 256, 0, p->stream>>>((const float *) buf, p->d_out, p->n);
-	GP_HIP(hipGetLastError());
-	if (p->d_inv) {
-		const uint32_t go = std::max<uint32_t>(1, std::min<uint32_t>(1024, (p->nv_orig + 255) / 256));
-		k_from_positions<<<go, 256, 0, p->stream>>>(p->d_out, p->d_inv, p->nv_orig, p->d_orig);
-		GP_HIP(hipGetLastError());
-		GP_HIP(hipMemcpyAsync(dist, p->d_orig, sizeof(double) * p->nv_orig, hipMemcpyDeviceToHost, p->stream));
-		GP_HIP(hipStreamSynchronize(p->stream));
-	} else if (p->coal) {
-		std::vector<double> tmp(p->n);
-		GP_HIP(hipMemcpyAsync(tmp.data(), p->d_out, sizeof(double) * p->n, hipMemcpyDeviceToHost, p->stream));
-		GP_HIP(hipStreamSynchronize(p->stream));
-		for (uint32_t v = 0; v < p->nv_orig; v++) dist[v] = p->inv[v] != NIL ? tmp[p->inv[v]] : INFINITY;
-	} else {
-		GP_HIP(hipMemcpyAsync(dist, p->d_out, sizeof(double) * p->n, hipMemcpyDeviceToHost, p->stream));
-		GP_HIP(hipStreamSynchronize(p->stream));
-	}
-	return GP_OK;
+		return result_out<double, double>(p->stream, (const double *) buf, p->d_inv, p->nv_orig, (double) INFINITY, dist);
+	return result_out<float, double>(p->stream, (const float *) buf, p->d_inv, p->nv_orig, (double) INFINITY, dist);
 }
 
 int plan_clusters(gp_plan *p, uint32_t *out)
@@ -1081,15 +1101,7 @@ int plan_clusters(gp_plan *p, uint32_t *out)
 	const uint32_t d = p->h_state->final_d;
 	const bool last_read = p->opts.result_buffer == GP_RESULT_LAST_READ;
 	const uint32_t *buf = (last_read ? !d : d) ? p->d_cl1 : p->d_cl0;
-	std::vector<uint32_t> tmp(p->n);
-	GP_HIP(hipMemcpyAsync(tmp.data(), buf, 4ull * p->n, hipMemcpyDeviceToHost, p->stream));
-	GP_HIP(hipStreamSynchronize(p->stream));
-	if (p->coal) {
-		for (uint32_t v = 0; v < p->nv_orig; v++) out[v] = p->inv[v] != NIL ? tmp[p->inv[v]] : GP_NIL;
-	} else {
-		std::memcpy(out, tmp.data(), 4ull * p->n);
-	}
-	return GP_OK;
+	return result_out<uint32_t, uint32_t>(p->stream, buf, p->d_inv, p->nv_orig, GP_NIL, out);
 }
 
 int plan_trace(gp_plan *p, uint32_t *out, uint32_t cap, uint32_t *n)
@@ -1352,16 +1364,10 @@ int ptp_iter_error(Che *mesh, const uint32_t *src, uint32_t ns, const double *ex
 	// Exact distances in the plan's ring numbering (test_geodesics_ptp_coalescence.cu:37).
 	std::vector<double> exc(nv);
 	for (uint32_t v = 0; v < nv; v++) exc[p->inv[v]] = exact[v];
-	double *d_exact = nullptr, *d_acc = nullptr;
-	struct Free {
-		std::vector<void *> v;
-		~Free() { for (void *q : v) (void) hipFree(q); }
-	} fr;
-	if (hipMalloc(&d_exact, 8ull * nv) != hipSuccess || hipMalloc(&d_acc, 8) != hipSuccess) {
-		fr.v = { d_exact, d_acc };
+	PoolBuf<double> exactb(p->stream), accb(p->stream);
+	if (exactb.alloc(8ull * nv) != hipSuccess || accb.alloc(8) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "iter_error: allocation failed");
-	}
-	fr.v = { d_exact, d_acc };
+	double *const d_exact = exactb.p, *const d_acc = accb.p;
 	GP_HIP(hipMemcpy(d_exact, exc.data(), 8ull * nv, hipMemcpyHostToDevice));
 	const uint32_t ig = std::max<uint32_t>(1, std::min<uint32_t>(1024, (p->n + 255) / 256));
 	const uint32_t done0 = p->nl < 3 ? 1u : 0u;

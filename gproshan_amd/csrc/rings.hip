@@ -255,12 +255,13 @@ static uint32_t fill_grid(uint32_t n) { return std::max<uint32_t>(1, std::min<ui
 constexpr uint32_t ORDER_LDS_SMALL = 1024, ORDER_LDS = 12288;
 
 int RingOrder::queue(const Levels &lv, const LevelInfo &li, const uint32_t *limits, const uint32_t *inv,
-                     const uint32_t *d_src, uint32_t ns, hipStream_t stream)
+                     const uint32_t *d_src, uint32_t ns, hipStream_t on)
 {
+	stream = on;
 	const bool wide = li.max_ring > ORDER_LDS;
-	if (hipMalloc(&child, 4ull * CHILD_ROWS * li.nr) != hipSuccess || hipMalloc(&rank0, 4ull * ns) != hipSuccess ||
-	    hipMalloc(&out, 4ull * lv.nv) != hipSuccess ||
-	    (wide && hipMalloc(&work, 16ull * li.max_ring) != hipSuccess))
+	if (pool_malloc(&child, 4ull * CHILD_ROWS * li.nr) != hipSuccess || pool_malloc(&rank0, 4ull * ns) != hipSuccess ||
+	    pool_malloc(&out, 4ull * lv.nv) != hipSuccess ||
+	    (wide && pool_malloc(&work, 16ull * li.max_ring) != hipSuccess))
 		return fail(GP_ERR_NOMEM, "rings: device allocation failed");
 	const DeviceMesh *dm = lv.dm;
 	const OrderArgs a{ lv.sorted, limits, lv.level, inv, dm->fan_off, dm->fan, dm->closed, li.nl, li.nr, child, rank0, out };
@@ -306,10 +307,10 @@ static int toplesets_bfs(Che &m, const uint32_t *src, uint32_t ns, uint32_t *lev
 		std::vector<void *> p;
 		~Free() { for (void *q : p) (void) hipFree(q); }
 	} fr;
-	if (hipMalloc(&d_level, 4ull * nv) != hipSuccess || hipMalloc(&d_sorted, 4ull * nv) != hipSuccess ||
-	    hipMalloc(&d_limits, 4ull * (nv + 2)) != hipSuccess || hipMalloc(&d_nl, 4) != hipSuccess ||
-	    hipMalloc(&d_src, 4ull * ns) != hipSuccess || hipMalloc(&d_key, 8ull * nv) != hipSuccess ||
-	    hipMalloc(&d_job, sizeof(BfsJob)) != hipSuccess) {
+	if (device_malloc(&d_level, 4ull * nv) != hipSuccess || device_malloc(&d_sorted, 4ull * nv) != hipSuccess ||
+	    device_malloc(&d_limits, 4ull * (nv + 2)) != hipSuccess || device_malloc(&d_nl, 4) != hipSuccess ||
+	    device_malloc(&d_src, 4ull * ns) != hipSuccess || device_malloc(&d_key, 8ull * nv) != hipSuccess ||
+	    device_malloc(&d_job, sizeof(BfsJob)) != hipSuccess) {
 		fr.p = { d_level, d_sorted, d_limits, d_nl, d_src, d_key, d_job };
 		return fail(GP_ERR_NOMEM, "toplesets_gpu: allocation failed");
 	}
@@ -348,14 +349,13 @@ int toplesets_gpu(Che &m, const uint32_t *src, uint32_t ns, uint32_t *levels, ui
 	int rc = upload_mesh(m);
 	if (rc) return rc;
 	const uint32_t nv = m.nv;
-	hipStream_t stream = nullptr;
-	GP_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-	std::unique_ptr<std::remove_pointer<hipStream_t>::type, hipError_t (*)(hipStream_t)> sg(stream, hipStreamDestroy);
-	uint32_t *d_src = nullptr, *d_inv = nullptr;
-	if (hipMalloc(&d_src, 4ull * ns) != hipSuccess) return fail(GP_ERR_NOMEM, "toplesets_gpu: allocation failed");
-	std::unique_ptr<uint32_t, hipError_t (*)(void *)> g0(d_src, hipFree);
-	if (hipMalloc(&d_inv, 4ull * nv) != hipSuccess) return fail(GP_ERR_NOMEM, "toplesets_gpu: allocation failed");
-	std::unique_ptr<uint32_t, hipError_t (*)(void *)> g1(d_inv, hipFree);
+	PoolStream ps;
+	GP_HIP(ps.create());
+	const hipStream_t stream = ps.s;
+	PoolBuf<uint32_t> srcb(stream), invb(stream);
+	if (srcb.alloc(4ull * ns) != hipSuccess || invb.alloc(4ull * nv) != hipSuccess)
+		return fail(GP_ERR_NOMEM, "toplesets_gpu: allocation failed");
+	uint32_t *const d_src = srcb.p, *const d_inv = invb.p;
 	GP_HIP(hipMemcpy(d_src, src, 4ull * ns, hipMemcpyHostToDevice));
 	Levels lv;
 	if ((rc = lv.create(m.dev, stream))) return rc;
