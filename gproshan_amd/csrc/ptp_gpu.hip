@@ -756,15 +756,14 @@ static int result_out(hipStream_t stream, const T *buf, const uint32_t *inv, uin
 	return GP_OK;
 }
 
-// From this many vertices the host's BFS (30 ns a vertex once its tables leave
-// the caches) takes longer than the solve it runs beside: 1M vertices in FP64
-// 29.3 ms with the host's order, 22.8 with the device's; 615k 14.3 against 15.2,
-// 201k in FP32 3.6 against 4.3.
-constexpr uint32_t ORDER_MIN_NV = 900000;
-
+// The sorted order beside the solve, from the plan's own rings on a second
+// stream, where a host BFS on a thread took 30 ns a vertex once its tables left
+// the caches: 1M vertices in FP64 27.3 ms with the host's order, 18.6 with the
+// device's; 615k in FP32 12.2 against 7.5, 201k of 16 sources 3.17 against 2.13,
+// 10k 0.86 against 0.80 (201k of one source, 517 rings: 4.12 against 4.23).
 bool plan_order_possible(const Che &m, const gp_ptp_opts &o)
 {
-	return m.nv >= ORDER_MIN_NV && m.manifold && o.device_setup && o.schedule == GP_SCHED_RINGS && o.coalesce && !o.clusters &&
+	return m.manifold && o.device_setup && o.schedule == GP_SCHED_RINGS && o.coalesce && !o.clusters &&
 	       m.max_link <= std::min(MAXS, ORDER_MAX_LINK);
 }
 

@@ -214,7 +214,7 @@ def ptp(mesh, sources, *, precision=L.PREC_F32, result_buffer=L.RESULT_LAST_WRIT
         coalesce=True, tol=PTP_TOL, max_sweeps=0, grid=0, launch_mode=L.LAUNCH_GRAPH, uncapped=False,
         device_setup=False, fp32_geometry=L.GEO_AUTO):
     """One PTP solve with explicit options; returns (dist, sorted, stats dict).
-    sorted is the reference's BFS order, built on the host while the solve runs."""
+    sorted is the reference's BFS order, built while the solve runs."""
     src = _u32(sources)
     o = L.default_opts(precision=precision, result_buffer=result_buffer, schedule=schedule,
                        coalesce=int(coalesce), tol=tol, max_sweeps=max_sweeps, grid=grid,
