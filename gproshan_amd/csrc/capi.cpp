@@ -205,7 +205,7 @@ static int ptp_gpu_driver(gp_che *mesh, const uint32_t *sources, uint32_t ns, co
 	o.coalesce = coalesce;
 	o.clusters = clusters ? 1 : 0;
 	gp_plan *p = nullptr;
-	int rc = gp::plan_create_rings(&mesh->m, sources, ns, limits, nl, sorted, o, &p);
+	int rc = gp::plan_create_given(&mesh->m, sources, ns, limits, nl, sorted, o, &p);
 	if (rc) return rc;
 	std::unique_ptr<gp_plan, void (*)(gp_plan *)> guard(p, gp_plan_destroy);
 	gp_ptp_stats st{};

@@ -179,6 +179,10 @@ int plan_create_rings(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_
 int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp_opts &opts, gp_plan **out,
                        const double *dhat = nullptr, double width = 0, gp_mlp *mlp = nullptr,
                        bool want_order = false);
+// Plan of the caller's rings, its tables built on the device where that gives the
+// same sweeps.
+int plan_create_given(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_t *limits, uint32_t nl,
+                      const uint32_t *sorted, const gp_ptp_opts &opts, gp_plan **out);
 // Whether a plan of these options, made with want_order, works out the
 // reference's order (sorted) on the device, and that order (waits for it; have =
 // false: the plan has none).

@@ -195,12 +195,20 @@ __global__ __launch_bounds__(1024) void k_compact_limits(uint32_t *limits, uint3
 	if (threadIdx.x == 0) *nl = carry;
 }
 
+// (src_pos null: k_source_positions)
 __global__ void k_positions(const uint32_t *sorted, uint32_t nr, uint32_t *inv, uint32_t *src_pos, uint32_t ns)
 {
 	for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < nr; q += gridDim.x * blockDim.x) {
 		inv[sorted[q]] = q;
-		if (q < ns) src_pos[q] = q;
+		if (src_pos && q < ns) src_pos[q] = q;
 	}
+}
+
+// The sources' positions in the caller's order (a label is an index into it).
+__global__ void k_source_positions(const uint32_t *inv, const uint32_t *src, uint32_t ns, uint32_t *src_pos)
+{
+	const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
+	if (q < ns) src_pos[q] = inv[src[q]];
 }
 
 }  // namespace gp
@@ -353,17 +361,14 @@ static bool ring_like(int schedule)
 	       schedule == GP_SCHED_RING_BAND;
 }
 
-// Builds a plan from given rings (limits/sorted in the original numbering;
-// for the band schedules, the bands in the order to sweep them).
-int plan_create_rings(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_t *limits, uint32_t nl,
-                      const uint32_t *sorted, const gp_ptp_opts &opts, gp_plan **out)
+// The kernels index with the caller's rings: checks them all on the host.
+static int check_rings(const Che *mesh, const uint32_t *src, uint32_t ns, const uint32_t *limits, uint32_t nl,
+                       const uint32_t *sorted)
 {
-	*out = nullptr;
 	if (!mesh || !src || !limits || !sorted) return fail(GP_ERR_INVALID, "plan: null argument");
 	if (ns == 0 || nl < 2) return fail(GP_ERR_INVALID, "plan: no sources / empty rings");
 	const uint32_t nr = limits[nl - 1];
 	if (nr > mesh->nv) return fail(GP_ERR_INVALID, "plan: limits exceed the vertex count");
-	// The kernels index with these values: check them all on the host.
 	if (limits[0] != 0) return fail(GP_ERR_INVALID, "plan: limits[0] must be 0");
 	for (uint32_t q = 1; q < nl; q++)
 		if (limits[q] < limits[q - 1]) return fail(GP_ERR_INVALID, "plan: limits must be non-decreasing");
@@ -371,6 +376,17 @@ int plan_create_rings(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_
 		if (sorted[q] >= mesh->nv) return fail(GP_ERR_INVALID, "plan: sorted[%u] out of range", q);
 	for (uint32_t q = 0; q < ns; q++)
 		if (src[q] >= mesh->nv) return fail(GP_ERR_INVALID, "plan: source %u out of range", src[q]);
+	return GP_OK;
+}
+
+// Builds a plan from given rings (limits/sorted in the original numbering;
+// for the band schedules, the bands in the order to sweep them).
+int plan_create_rings(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_t *limits, uint32_t nl,
+                      const uint32_t *sorted, const gp_ptp_opts &opts, gp_plan **out)
+{
+	*out = nullptr;
+	if (const int bad = check_rings(mesh, src, ns, limits, nl, sorted)) return bad;
+	const uint32_t nr = limits[nl - 1];
 	if (opts.precision != GP_PREC_F32 && opts.precision != GP_PREC_F64)
 		return fail(GP_ERR_INVALID, "plan: unknown precision %d", opts.precision);
 	if (!ring_like(opts.schedule)) return fail(GP_ERR_INVALID, "plan_create_rings: ring or band schedule only");
@@ -575,17 +591,24 @@ __global__ void k_max_level(const uint32_t *level, uint32_t n, uint32_t *out)
 	if ((threadIdx.x & 63u) == 0 && m) atomicMax(out, m);
 }
 
-int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp_opts &opts, gp_plan **out,
-                       const double *dhat, double width, gp_mlp *mlp, bool want_order)
+// Rings from the caller: the ring of each vertex (NIL: in none) and the limits.
+struct GivenRings {
+	const uint32_t *limits;
+	uint32_t nl;
+	std::vector<uint32_t> ring;
+};
+
+static int create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp_opts &opts, gp_plan **out,
+                         const double *dhat, double width, gp_mlp *mlp, bool want_order, const GivenRings *given)
 {
 	*out = nullptr;
 	if (!mesh || !src) return fail(GP_ERR_INVALID, "plan: null argument");
 	if (ns == 0) return fail(GP_ERR_INVALID, "plan: no sources");
-	if (!ring_like(opts.schedule) || !opts.coalesce || opts.clusters)
+	if (!ring_like(opts.schedule) || !opts.coalesce || (opts.clusters && !given))
 		return fail(GP_ERR_INVALID, "plan_create_device: ring or band schedule, coalesced, without labels only");
 	if (opts.precision != GP_PREC_F32 && opts.precision != GP_PREC_F64)
 		return fail(GP_ERR_INVALID, "plan: unknown precision %d", opts.precision);
-	{
+	if (!given) {
 		std::vector<uint8_t> seen(mesh->nv, 0);
 		for (uint32_t q = 0; q < ns; q++) {
 			if (src[q] >= mesh->nv) return fail(GP_ERR_INVALID, "plan: source %u out of range", src[q]);
@@ -618,9 +641,13 @@ int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp
 	if ((rc = upload(p->d_srcv, srcv))) return rc;
 	uint32_t *const d_srcv = p->d_srcv;
 	lv.clear();
-	lv.seed(d_srcv, 0, ns);
-	if ((rc = lv.expand())) return rc;
-	if (dhat || mlp) {
+	lv.seed(d_srcv, 0, given ? 0u : ns);
+	if (given) {
+		GP_HIP(hipMemcpyAsync(lv.level, given->ring.data(), 4ull * mesh->nv, hipMemcpyHostToDevice, p->stream));
+		lv.sort();
+	} else if ((rc = lv.expand())) {
+		return rc;
+	} else if (dhat || mlp) {
 		// Bands of dhat in place of the BFS levels of the reached vertices:
 		// the caller's dhat, or the network's prediction from these levels
 		// (the features' ring index), kept on the device.
@@ -656,7 +683,8 @@ int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp
 	}
 	LevelInfo li;
 	if ((rc = lv.info(li))) return rc;
-	const uint32_t nl = li.nl, nr = li.nr, rows = li.rows;
+	// Given rings may end in empty ones, which the sort doesn't see.
+	const uint32_t nl = given ? given->nl : li.nl, nr = li.nr, rows = li.rows;
 	p->nl = nl;
 	p->nr = nr;
 	p->n = nr;
@@ -681,14 +709,18 @@ int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp
 	           pool_malloc(&p->d_cgeo64, sizeof(double4) * std::max<size_t>(lanes, 1)) != hipSuccess) {
 		return fail(GP_ERR_NOMEM, "plan: device allocation failed");
 	}
-	GP_HIP(hipMemcpyAsync(p->d_limits, lv.limits, 4ull * nl, hipMemcpyDeviceToDevice, p->stream));
+	if (given)
+		GP_HIP(hipMemcpyAsync(p->d_limits, given->limits, 4ull * nl, hipMemcpyHostToDevice, p->stream));
+	else
+		GP_HIP(hipMemcpyAsync(p->d_limits, lv.limits, 4ull * nl, hipMemcpyDeviceToDevice, p->stream));
 	GP_HIP(hipMemcpyAsync(p->d_coff, lv.coff, 4ull * (p->nchunks + 1), hipMemcpyDeviceToDevice, p->stream));
 	const uint32_t g = std::max<uint32_t>(1, std::min<uint32_t>(2048, (mesh->nv + 255) / 256));
 	k_fill_u32<<<g, 256, 0, p->stream>>>(p->d_inv, mesh->nv, GP_NIL);
-	k_positions<<<g, 256, 0, p->stream>>>(lv.sorted, nr, p->d_inv, p->d_src, ns);
+	k_positions<<<g, 256, 0, p->stream>>>(lv.sorted, nr, p->d_inv, given ? nullptr : p->d_src, ns);
+	if (given) k_source_positions<<<(ns + 255) / 256, 256, 0, p->stream>>>(p->d_inv, d_srcv, ns, p->d_src);
 	const uint32_t npos = p->nchunks * 64;
 	const uint32_t gg = std::max<uint32_t>(1, std::min<uint32_t>(4096, (npos + 255) / 256));
-	const uint32_t *nr_at = lv.limits + (nl - 1);
+	const uint32_t *nr_at = lv.limits + (li.nl - 1);
 	if (f64)
 		k_gather_tables<true, false><<<gg, 256, 0, p->stream>>>(lv.sorted, p->d_inv, nr_at, npos, S, lv.coff, mt,
 		                                                         p->d_cid, nullptr, nullptr, nullptr, p->d_cx64);
@@ -707,6 +739,56 @@ int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp
 	if ((rc = plan_run_buffers(p.get(), f64))) return rc;
 	*out = p.release();
 	return GP_OK;
+}
+
+int plan_create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_ptp_opts &opts, gp_plan **out,
+                       const double *dhat, double width, gp_mlp *mlp, bool want_order)
+{
+	return create_device(mesh, src, ns, opts, out, dhat, width, mlp, want_order, nullptr);
+}
+
+// The ring of each vertex, if the rings can be swept from device-built tables:
+// no vertex twice, every source and every neighbour of a ring vertex in a ring
+// (then the sweeps over the whole mesh and those over its reached faces read
+// the same values), a manifold mesh (fans keep their order when it is rebuilt
+// from the reached faces).
+static bool rings_closed(const Che &m, const uint32_t *src, uint32_t ns, const uint32_t *sorted, GivenRings &g)
+{
+	const uint32_t nr = g.limits[g.nl - 1];
+	if (!m.manifold || nr == 0 || g.nl > m.nv + 1) return false;
+	g.ring.assign(m.nv, NIL);
+	for (uint32_t r = 0; r + 1 < g.nl; r++)
+		for (uint32_t q = g.limits[r]; q < g.limits[r + 1]; q++) {
+			if (g.ring[sorted[q]] != NIL) return false;
+			g.ring[sorted[q]] = r;
+		}
+	for (uint32_t q = 0; q < ns; q++)
+		if (g.ring[src[q]] == NIL) return false;
+	if (nr == m.nv) return true;
+	for (uint32_t q = 0; q < nr; q++)
+		for (uint32_t k = m.fan_off[sorted[q]]; k < m.fan_off[sorted[q] + 1]; k++)
+			if (g.ring[m.fan[k]] == NIL) return false;
+	return true;
+}
+
+// Plan of given rings: the tables gathered on the device where that reads the
+// same values, else laid out on the host.  77k vertices, 16 sources, FP64 with
+// labels, from the sources to the labels: 8.4 ms with rings and tables built on
+// the host, 2.5 with both built on the device.
+int plan_create_given(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_t *limits, uint32_t nl,
+                      const uint32_t *sorted, const gp_ptp_opts &opts, gp_plan **out)
+{
+	*out = nullptr;
+	if (const int bad = check_rings(mesh, src, ns, limits, nl, sorted)) return bad;
+	GivenRings g{ limits, nl, {} };
+	if (rings_closed(*mesh, src, ns, sorted, g)) {
+		gp_ptp_opts o = opts;
+		o.coalesce = 1;
+		const int rd = create_device(mesh, src, ns, o, out, nullptr, 0, nullptr, false, &g);
+		if (rd != GP_ERR_CAPACITY) return rd;
+		clear_error();   // a fan too long for the device build
+	}
+	return plan_create_rings(mesh, src, ns, limits, nl, sorted, opts, out);
 }
 
 // n values in the caller's numbering into host memory: written by the device to

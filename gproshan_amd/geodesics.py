@@ -394,7 +394,7 @@ class geodesics:
         elif opt == self.PTP_GPU and cluster:
             # The reference's GPU drivers with their cluster output
             # (src/geodesics.cpp:225-240).
-            ts = mesh.compute_toplesets(src)
+            ts = mesh.compute_toplesets(src, gpu=True)
             drv = parallel_toplesets_propagation_coalescence_gpu if len(src) == 1 else parallel_toplesets_propagation_gpu
             d, _, cl = drv(mesh, src, ts, clusters=True)
             self._sorted[:] = ts[1]
