@@ -1,5 +1,5 @@
 // Batched PTP: many (mesh, source) fields of uneven size in one persistent
-// launch (a hipGraph of its queue reset and the kernel).
+// launch behind the reset of its queue.
 //
 // Each 1024-thread workgroup repeatedly takes the next job from an atomic
 // queue (jobs sorted by decreasing cost V^1.5, so the grid drains evenly), and
@@ -24,17 +24,19 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <numeric>
 #include <vector>
 
 #include "device.hpp"
+#include "levels.hpp"
 #include "rings_dev.hpp"
 #include "sweep_dev.hpp"
 
 namespace gp {
 
 struct BMesh {
-	const uint32_t *fan_off, *fan;
+	const uint32_t *fan_off, *fan, *link8;
 	const uint8_t *closed;
 	const uint32_t *coff, *cid;
 	const float2 *cgeo;
@@ -65,7 +67,16 @@ struct BArgs {
 	uint32_t *fcid, *fmidx, *finv;
 	float2 *fgeo;
 	size_t fslots;
+	uint32_t bit_words;   // LDS words of the BFS's visited bits; 0: bfs_block
 };
+
+// Pointers that the kernel reads from memory: without the address space their
+// loads are flat ones, which wait for LDS too.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(1))) T *in_global(const T *p)
+{
+	return (const __attribute__((address_space(1))) T *) p;
+}
 
 // The field's tables as relax_lane reads them.
 struct FieldTables {
@@ -78,17 +89,160 @@ struct FieldTables {
 
 __global__ void k_batch_reset(uint32_t *queue) { *queue = 0; }
 
-// NT threads per field (a multiple of 64, at most 1024).
-template <uint32_t NT, uint32_t MS>
-__global__ __launch_bounds__(NT) void k_batch(BArgs a)
+// Barrier for data in LDS: stores to memory stay in flight (__syncthreads waits
+// for them).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// BFS of one source by the whole workgroup: rings, limits and the vertices'
+// positions.  The visited bits and the frontier are in LDS, eight lanes expand a
+// vertex from its 32-byte link row, so a level is one round trip to the row and
+// two LDS barriers; frontiers past BQ vertices are read back from sorted[].  No
+// value depends on the order inside a ring, but it follows the frontier's (the
+// waves' counts are scanned), so that the 64 vertices of a chunk lie side by side
+// and a sweep's neighbour loads share their lines.  The ordered BFS (bfs_block)
+// reads each level's links twice and keys every neighbour with a 64-bit atomic in
+// memory: with the gather of the tables 7.9 of the 30.1 ms of 1,024 fields of
+// 2k-58k vertices (1,024 threads a field), now 1.9 of 26.7.
+constexpr uint32_t BQ = 1024, BFS_UNROLL = 4;   // BQ: whole passes of the loop below
+constexpr uint32_t MAX_BIT_WORDS = 8192;        // 32 KB: meshes to 262,144 vertices
+
+template <uint32_t NT>
+__device__ __forceinline__ uint32_t bfs_bits(const BMesh &M, uint32_t src, uint32_t *bits, uint32_t (*s_q)[BQ],
+                                             uint32_t *s_cnt, uint32_t *s_end, uint32_t *sorted, uint32_t *inv,
+                                             uint32_t *limits)
 {
-	__shared__ uint32_t s_job, s_bad;
+	constexpr uint32_t GROUPS = NT / LINK_ROW, NW = NT / 64;
+	static_assert(BQ % (GROUPS * BFS_UNROLL) == 0, "a pass reads the frontier from one place");
+	static_assert(NW * BFS_UNROLL <= 64, "one lane a count");
+	const uint32_t tid = threadIdx.x, lane = tid & 63u, slot = tid % LINK_ROW, group = tid / LINK_ROW;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const auto *link8 = in_global(M.link8);
+	for (uint32_t w = tid; w < (M.nv + 31) / 32; w += NT) bits[w] = 0;
+	__syncthreads();
+	if (tid == 0) {
+		bits[src >> 5] = 1u << (src & 31u);
+		s_q[0][0] = src;
+		sorted[0] = src;
+		inv[src] = 0;
+		limits[0] = 0;
+		limits[1] = 1;
+	}
+	__syncthreads();
+	uint32_t fb = 0, fe = 1, nl = 2;   // the frontier is sorted[fb, fe)
+	for (uint32_t cur = 0;; cur ^= 1u) {
+		const uint32_t n = fe - fb;
+		uint32_t p = fe;               // the next ring is sorted[fe, p)
+		auto claim = [&](uint32_t u) -> bool {
+			const uint32_t bit = 1u << (u & 31u);
+			return u != GP_NIL && !(atomicOr(&bits[u >> 5], bit) & bit);
+		};
+		auto append = [&](uint32_t u, uint32_t at) {
+			if (at - fe < BQ) s_q[cur ^ 1u][at - fe] = u;
+			sorted[at] = u;
+			inv[u] = at;
+		};
+		for (uint32_t c0 = 0; c0 < n; c0 += GROUPS * BFS_UNROLL) {
+			uint32_t id[BFS_UNROLL];
+			unsigned long long got[BFS_UNROLL];
+			uint32_t more = 0;         // bit r: the link of pass r goes on (lane of entry 7)
+#pragma unroll
+			for (uint32_t r = 0; r < BFS_UNROLL; r++) {
+				const uint32_t c = c0 + r * GROUPS + group;
+				id[r] = GP_NIL;
+				if (c < n) {
+					uint32_t v;
+					if (c0 < BQ) v = s_q[cur][c];
+					else v = sorted[fb + c];
+					id[r] = link8[(size_t) v * LINK_ROW + slot];
+				}
+			}
+#pragma unroll
+			for (uint32_t r = 0; r < BFS_UNROLL; r++) {
+				if (id[r] != GP_NIL && (id[r] & LONG_LINK)) {
+					id[r] &= ~LONG_LINK;
+					more |= 1u << r;
+				}
+				got[r] = __ballot(claim(id[r]));
+				if (lane == 0) s_cnt[r * NW + wave] = (uint32_t) __popcll(got[r]);
+				if (more >> r & 1u) s_cnt[r * NW + wave] = (uint32_t) __popcll(got[r]) | LONG_LINK;
+			}
+			lds_barrier();
+			// Every wave scans the pass's counts, one a lane.
+			uint32_t x = lane < NW * BFS_UNROLL ? s_cnt[lane] : 0u;
+			const bool any_more = __ballot((x & LONG_LINK) != 0u) != 0;
+			x &= ~LONG_LINK;
+			uint32_t inc = x;
+			for (uint32_t o = 1; o < 64; o <<= 1) {
+				const uint32_t y = __shfl_up(inc, o);
+				if (lane >= o) inc += y;
+			}
+#pragma unroll
+			for (uint32_t r = 0; r < BFS_UNROLL; r++) {
+				const uint32_t at = p + __shfl(inc - x, (int) (r * NW + wave));
+				if (got[r] >> lane & 1ull) append(id[r], at + (uint32_t) __popcll(got[r] & ((1ull << lane) - 1)));
+			}
+			p += __shfl(inc, 63);
+			if (any_more) {
+				// The entries past eight, from the fan table, as they come.
+				if (tid == 0) *s_end = p;
+				lds_barrier();
+				for (uint32_t r = 0; r < BFS_UNROLL; r++) {
+					uint32_t k = 0, e = 0;
+					if (__shfl((int) more, (int) (lane | (LINK_ROW - 1))) >> r & 1) {
+						const uint32_t c = c0 + r * GROUPS + group;
+						uint32_t v;
+						if (c0 < BQ) v = s_q[cur][c];
+						else v = sorted[fb + c];
+						k = M.fan_off[v] + LINK_ROW + slot;
+						e = M.fan_off[v + 1] - (M.closed[v] ? 1u : 0u);
+					}
+					for (; __ballot(k < e); k += LINK_ROW) {
+						const uint32_t u = k < e ? M.fan[k] & ID_MASK : GP_NIL;
+						const bool take = claim(u);
+						const unsigned long long m = __ballot(take);
+						if (!m) continue;
+						const int first = __builtin_ctzll(m);
+						uint32_t at = 0;
+						if (lane == (uint32_t) first) at = atomicAdd(s_end, (uint32_t) __popcll(m));
+						at = __shfl(at, first) + (uint32_t) __popcll(m & ((1ull << lane) - 1));
+						if (take) append(u, at);
+					}
+				}
+				lds_barrier();
+				p = __builtin_amdgcn_readfirstlane(*s_end);
+			}
+			lds_barrier();
+		}
+		if (p == fe) break;
+		if (p - fe > BQ) __syncthreads();   // sorted[] is read back
+		fb = fe;
+		fe = p;
+		if (tid == 0) limits[nl] = fe;
+		nl++;
+	}
+	__syncthreads();
+	return nl;
+}
+
+// NT threads per field (a multiple of 64, at most 1024).
+//
+// The sweeps, 25 of 27 ms, run 16 waves a CU (128 registers a lane), each taking
+// one chunk after the other: rows from memory (43 GB in all; 79 % of the requests
+// miss L2, as 32 fields share one), neighbours' values, ~510 vector instructions
+// (the units are busy 46 % of the time), a chain that four waves a SIMD cover in
+// part.  Two fields a CU of 512 threads take longer (38 ms) as they need twice
+// the cache, and asking for a chunk's rows one chunk ahead does too (29 ms).
+constexpr uint32_t BL = 1024;   // ring limits kept in LDS
+
+template <uint32_t NT, uint32_t MS>
+__global__ __launch_bounds__(NT, 4) void k_batch(BArgs a)
+{
+	extern __shared__ uint32_t s_bits[];
+	__shared__ uint32_t s_job, s_bad[3], s_cnt[64], s_end, s_q[2][BQ], s_lim[BL];
 	const uint32_t tid = threadIdx.x, nt = NT, wg = blockIdx.x;
 	const size_t mv = a.max_nv;
-	uint32_t *level = a.level + wg * mv;
 	uint32_t *sorted = a.sorted + wg * mv;
 	uint32_t *limits = a.limits + wg * (mv + 2);
-	unsigned long long *key = a.key + wg * mv;
 	float *d0 = a.dist + 2 * wg * mv, *d1 = d0 + mv;
 	uint32_t *fcid = a.fcid + wg * a.fslots, *fmidx = a.fmidx + wg * a.fslots, *finv = a.finv + wg * mv;
 	float2 *fgeo = a.fgeo + wg * a.fslots;
@@ -103,59 +257,83 @@ __global__ __launch_bounds__(NT) void k_batch(BArgs a)
 		const uint32_t job = __builtin_amdgcn_readfirstlane(s_job);
 		__syncthreads();
 		if (job >= a.njobs) break;
-		const uint32_t src = a.jobs[job].source;
 		const BMesh M = a.meshes[a.jobs[job].mesh];
 		const uint32_t nv = M.nv;
 		for (uint32_t v = tid; v < nv; v += nt) {
-			level[v] = GP_NIL; key[v] = ~0ull; sorted[v] = GP_NIL; finv[v] = GP_NIL;
+			finv[v] = GP_NIL;
 			d0[v] = INFINITY; d1[v] = INFINITY;
 		}
 		__syncthreads();
-		const BfsJob bj{ &a.jobs[job].source, 1u, level, key, sorted, limits, a.nlim + wg };
-		bfs_block(M.fan_off, M.fan, M.closed, bj);
-		const uint32_t nl = __hip_atomic_load(a.nlim + wg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		uint32_t nl;
+		if (a.bit_words) {
+			nl = bfs_bits<NT>(M, a.jobs[job].source, s_bits, s_q, s_cnt, &s_end, sorted, finv, limits);
+		} else {
+			uint32_t *level = a.level + wg * mv;
+			unsigned long long *key = a.key + wg * mv;
+			for (uint32_t v = tid; v < nv; v += nt) { level[v] = GP_NIL; key[v] = ~0ull; sorted[v] = GP_NIL; }
+			__syncthreads();
+			const BfsJob bj{ &a.jobs[job].source, 1u, level, key, sorted, limits, a.nlim + wg };
+			bfs_block(M.fan_off, M.fan, M.closed, bj);
+			nl = __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.nlim + wg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+			for (uint32_t q = tid; q < limits[nl - 1]; q += nt) finv[sorted[q]] = q;
+		}
+		for (uint32_t q = tid; q < min(nl, BL); q += nt) s_lim[q] = limits[q];
+		auto lim = [&](uint32_t q) { return __builtin_amdgcn_readfirstlane(q < BL ? s_lim[q] : limits[q]); };
+		__syncthreads();
 		// The field's ring-ordered tables: position p holds vertex sorted[p]
 		// (the source is position 0).
-		const uint32_t nr = nl ? limits[nl - 1] : 0u;
-		for (uint32_t q = tid; q < nr; q += nt) finv[sorted[q]] = q;
-		__syncthreads();
+		const uint32_t nr = lim(nl - 1);
+		const auto *mcoff = in_global(M.coff), *mcid = in_global(M.cid);
+		const auto *mgeo = in_global(M.cgeo);
+		const auto *perm = in_global(M.perm);
 		const uint32_t S = M.ms, npos = (nr + 63u) & ~63u;
 		for (uint32_t q = tid; q < npos; q += nt) {
 			const size_t fb = (size_t) (q >> 6) * S * 64 + (q & 63u);
 			uint32_t mb = 0, n = 0;
 			if (q < nr) {
 				const uint32_t v = sorted[q];
-				mb = M.coff[v];
-				n = M.coff[v + 1] - mb;
+				mb = mcoff[v];
+				n = mcoff[v + 1] - mb;
 			}
-			for (uint32_t k = 0; k < S; k++) {
-				const size_t at = fb + 64 * (size_t) k;
-				if (k < n) {
-					const uint32_t id = M.cid[mb + k];
-					fcid[at] = finv[id & SLOT_ID_MASK] | (id & ~SLOT_ID_MASK);
-					fgeo[at] = M.cgeo[mb + k];
-					fmidx[at] = mb + k;
-				} else {
-					fcid[at] = q | SLOT_EMPTY;
-					fgeo[at] = make_float2(0.f, 0.f);
-					fmidx[at] = 0;
+			// Eight slots at a time: their ids, then the positions and the
+			// geometry they lead to, in flight together.
+			for (uint32_t k0 = 0; k0 < S; k0 += 8) {
+				uint32_t id[8], at[8], p[8];
+				float2 g[8];
+#pragma unroll
+				for (uint32_t k = 0; k < 8; k++) {
+					at[k] = k0 + k < n ? mb + k0 + k : 0u;
+					id[k] = mcid[at[k]];
+					if (k0 + k >= n) id[k] = 0;
 				}
+#pragma unroll
+				for (uint32_t k = 0; k < 8; k++) { p[k] = finv[id[k] & SLOT_ID_MASK]; g[k] = float2{ mgeo[at[k]].x, mgeo[at[k]].y }; }
+#pragma unroll
+				for (uint32_t k = 0; k < 8; k++)
+					if (k0 + k < S) {
+						const bool has = k0 + k < n;
+						const size_t to = fb + 64 * (size_t) (k0 + k);
+						fcid[to] = has ? p[k] | (id[k] & ~SLOT_ID_MASK) : q | SLOT_EMPTY;
+						fgeo[to] = has ? g[k] : make_float2(0.f, 0.f);
+						fmidx[to] = has ? at[k] : 0u;
+					}
 			}
 		}
 		if (tid == 0 && nr) { d0[0] = 0.f; d1[0] = 0.f; }
+		if (tid < 3) s_bad[tid] = 0;
 		__syncthreads();
 		const FieldTables F{ fcid, fgeo, GeoRemap64{ M.cgeo64, fmidx }, nullptr, M.h, M.inv_h };
-		uint32_t i = 1, j = 2, d = 0, iter = 0;
+		uint32_t i = 1, j = 2, d = 0, iter = 0, turn = 0;
 		unsigned long long relax = 0;
 		const uint32_t max_iter = nl << 1;
 		bool done = nl < 3;
+		// One barrier a sweep: the ring test counts into one of three words in
+		// turn, the word after next cleared meanwhile.
 		while (!done) {
 			const uint32_t ii = i < (j >> 1) ? (j >> 1) : i;
-			const uint32_t start = limits[ii], end = limits[j], cend = limits[ii + 1];
+			const uint32_t start = lim(ii), end = lim(j), cend = lim(ii + 1);
 			const float *od = d ? d1 : d0;
 			float *nd = d ? d0 : d1;
-			if (tid == 0) s_bad = 0;
-			__syncthreads();
 			uint32_t bad = 0;
 			for (uint32_t c = (start >> 6) + wave; c < ((end + 63u) >> 6); c += nwave) {
 				const uint32_t pos = (c << 6) + lane;
@@ -168,20 +346,21 @@ __global__ __launch_bounds__(NT) void k_batch(BArgs a)
 				}
 				bad += (uint32_t) __popcll(__ballot(lbad));
 			}
-			if (lane == 0 && bad) atomicAdd(&s_bad, bad);
+			if (lane == 0 && bad) atomicAdd(&s_bad[turn], bad);
 			__syncthreads();
-			const uint32_t nbad = __builtin_amdgcn_readfirstlane(s_bad);
+			const uint32_t nbad = __builtin_amdgcn_readfirstlane(s_bad[turn]);
+			turn = turn == 2 ? 0 : turn + 1;
+			if (tid == 0) s_bad[turn == 2 ? 0 : turn + 1] = 0;
 			relax += end - start;
 			i = ii + (nbad == 0 ? 1u : 0u);
 			if (j < nl - 1) j++;
 			d ^= 1u;
 			iter++;
 			done = !(i < j) || !(iter < max_iter);
-			__syncthreads();
 		}
 		const float *res = d ? d1 : d0;            // the buffer the last sweep wrote
 		float *out = a.out + a.jobs[job].out;
-		for (uint32_t v = tid; v < nv; v += nt) out[M.perm[v]] = finv[v] != GP_NIL ? res[finv[v]] : INFINITY;
+		for (uint32_t v = tid; v < nv; v += nt) out[perm[v]] = finv[v] != GP_NIL ? res[finv[v]] : INFINITY;
 		if (tid == 0) { a.jobs[job].sweeps = iter; a.jobs[job].relax = relax; }
 		__syncthreads();
 	}
@@ -203,6 +382,13 @@ struct gp_batch {
 	std::vector<unsigned long long> out_off;   // user job -> offset of its field
 	std::vector<uint32_t> job_nv;              // user job -> vertices
 	std::vector<uint32_t> slot_of;             // user job -> queue slot
+	// Read back under the lock: the fields of the last run around the one asked
+	// for, as the caller takes them, and the jobs' sweep counts.
+	std::mutex mu;
+	double *h_win = nullptr;
+	unsigned long long win_at = 0, next_at = 0;   // next_at: behind the field read last
+	uint32_t win_n = 0;
+	std::vector<gp::BJob> jobs;                // of the last run (empty: not read yet)
 	gp::BMesh *d_meshes = nullptr;
 	gp::BJob *d_jobs = nullptr;
 	uint32_t *d_queue = nullptr;
@@ -217,8 +403,7 @@ struct gp_batch {
 	unsigned long long total_out = 0;
 	double tol = GP_PTP_TOL;
 	hipStream_t stream = nullptr;
-	hipGraphExec_t graph = nullptr;     // null when graphs are disabled
-	gp::BArgs args{};                    // the persistent launch (without a graph)
+	gp::BArgs args{};
 	const void *fn = nullptr;
 	hipEvent_t e0 = nullptr, e1 = nullptr;
 
@@ -232,8 +417,6 @@ struct gp_batch {
 		d_dist = nullptr;
 		d_fcid = d_fmidx = d_finv = nullptr;
 		d_fgeo = nullptr;
-		if (graph) (void) hipGraphExecDestroy(graph);
-		graph = nullptr;
 	}
 	~gp_batch()
 	{
@@ -242,6 +425,7 @@ struct gp_batch {
 			for (void *p : { (void *) t.coff, (void *) t.cid, (void *) t.cgeo, (void *) t.cgeo64, (void *) t.perm })
 				(void) hipFree(p);
 		for (void *p : { (void *) d_meshes, (void *) d_jobs, (void *) d_queue, (void *) d_out }) (void) hipFree(p);
+		gp::pinned_free(h_win);
 		if (e0) (void) hipEventDestroy(e0);
 		if (e1) (void) hipEventDestroy(e1);
 		if (stream) (void) hipStreamDestroy(stream);
@@ -260,64 +444,54 @@ static int up(V *&dst, const V *src, size_t n)
 
 // Fields whose fans all fit 8 slots run the 8-slot register path.
 template <uint32_t NT>
-static int launch_shape(uint32_t njobs, bool ms8, uint32_t &grid, const void *&fn)
+static int launch_shape(uint32_t njobs, bool ms8, uint32_t lds, uint32_t &grid, const void *&fn)
 {
 	int dev = 0, ncu = 0, occ = 0;
 	GP_HIP(hipGetDevice(&dev));
 	GP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
 	fn = ms8 ? (const void *) k_batch<NT, 8> : (const void *) k_batch<NT, MAXS>;
-	GP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, NT, 0));
+	GP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, NT, lds));
 	grid = std::max<uint32_t>(1, std::min<uint32_t>(njobs, (uint32_t) ncu * (uint32_t) std::max(1, occ)));
 	return GP_OK;
 }
 
-// Sizes the per-workgroup scratch for `block` threads per field and captures
-// the queue reset + persistent launch into the batch's graph.
+// Sizes the per-workgroup scratch for `block` threads per field.
 static int batch_configure(gp_batch *b, uint32_t block)
 {
 	b->free_scratch();
 	uint32_t grid = 0;
 	const void *fn = nullptr;
 	int rc;
+	const uint32_t words = (b->max_nv + 31) / 32, bit_words = words <= MAX_BIT_WORDS ? words : 0;
 	switch (block) {
-	case 256: rc = launch_shape<256>(b->njobs, b->max_slots <= 8, grid, fn); break;
-	case 512: rc = launch_shape<512>(b->njobs, b->max_slots <= 8, grid, fn); break;
-	case 1024: rc = launch_shape<1024>(b->njobs, b->max_slots <= 8, grid, fn); break;
+	case 256: rc = launch_shape<256>(b->njobs, b->max_slots <= 8, 4 * bit_words, grid, fn); break;
+	case 512: rc = launch_shape<512>(b->njobs, b->max_slots <= 8, 4 * bit_words, grid, fn); break;
+	case 1024: rc = launch_shape<1024>(b->njobs, b->max_slots <= 8, 4 * bit_words, grid, fn); break;
 	default: return fail(GP_ERR_INVALID, "batch: block must be 256, 512 or 1024 (got %u)", block);
 	}
 	if (rc) return rc;
 	const size_t mv = b->max_nv;
 	// Field tables: the largest field's chunks at the longest fan's width.
 	const size_t fslots = ((mv + 63) / 64) * 64 * (size_t) b->max_slots;
-	const size_t per_wg = 4 * mv * 3 + 4 * (mv + 2) + 8 * mv + 8 * mv + fslots * (4 + 4 + sizeof(float2));
+	const size_t bfs_mv = bit_words ? 0 : mv;   // the ordered BFS's levels and keys
+	const size_t per_wg = 4 * mv * 2 + 4 * (mv + 2) + 12 * bfs_mv + 8 * mv + fslots * (4 + 4 + sizeof(float2));
 	// At most 32 GiB of scratch: a wider grid than that would take no more
 	// fields at once than the workgroups that fit.
 	const size_t cap = std::max<size_t>(1, (32ull << 30) / std::max<size_t>(per_wg, 1));
 	grid = (uint32_t) std::min<size_t>(grid, cap);
 	const size_t g = grid;
-	if (device_malloc(&b->d_level, 4 * mv * g) != hipSuccess || device_malloc(&b->d_sorted, 4 * mv * g) != hipSuccess ||
+	if (device_malloc(&b->d_level, std::max<size_t>(4, 4 * bfs_mv * g)) != hipSuccess || device_malloc(&b->d_sorted, 4 * mv * g) != hipSuccess ||
 	    device_malloc(&b->d_limits, 4 * (mv + 2) * g) != hipSuccess || device_malloc(&b->d_nlim, 4 * g) != hipSuccess ||
-	    device_malloc(&b->d_key, 8 * mv * g) != hipSuccess || device_malloc(&b->d_dist, 8 * mv * g) != hipSuccess ||
+	    device_malloc(&b->d_key, std::max<size_t>(8, 8 * bfs_mv * g)) != hipSuccess || device_malloc(&b->d_dist, 8 * mv * g) != hipSuccess ||
 	    device_malloc(&b->d_finv, 4 * mv * g) != hipSuccess || device_malloc(&b->d_fcid, 4 * fslots * g) != hipSuccess ||
 	    device_malloc(&b->d_fmidx, 4 * fslots * g) != hipSuccess || device_malloc(&b->d_fgeo, sizeof(float2) * fslots * g) != hipSuccess) {
 		b->free_scratch();
 		return fail(GP_ERR_NOMEM, "batch: scratch allocation failed (%u workgroups x %u vertices)", grid, b->max_nv);
 	}
 	BArgs a{ b->d_meshes, b->d_jobs, b->njobs, b->max_nv, b->d_queue, b->d_level, b->d_sorted, b->d_limits, b->d_nlim,
-	         b->d_key, b->d_dist, b->d_out, b->tol, b->d_fcid, b->d_fmidx, b->d_finv, b->d_fgeo, fslots };
+	         b->d_key, b->d_dist, b->d_out, b->tol, b->d_fcid, b->d_fmidx, b->d_finv, b->d_fgeo, fslots, bit_words };
 	b->args = a;
 	b->fn = fn;
-	b->grid = grid;
-	b->block = block;
-	if (!graphs_enabled()) return GP_OK;
-	void *kargs[] = { &a };
-	uint32_t *queue = b->d_queue;
-	void *rargs[] = { &queue };
-	GraphChain gc;
-	gc.add((const void *) k_batch_reset, dim3(1), dim3(1), rargs);
-	gc.add(fn, dim3(grid), dim3(block), kargs);
-	const hipError_t e = gc.instantiate(&b->graph);
-	if (e != hipSuccess) return fail(GP_ERR_HIP, "batch graph: %s", hipGetErrorString(e));
 	b->grid = grid;
 	b->block = block;
 	return GP_OK;
@@ -325,14 +499,14 @@ static int batch_configure(gp_batch *b, uint32_t block)
 
 static int batch_launch(gp_batch *b, float *ms)
 {
+	std::lock_guard<std::mutex> lock(b->mu);
+	b->win_n = 0;
+	b->next_at = 0;
+	b->jobs.clear();
 	GP_HIP(hipEventRecord(b->e0, b->stream));
-	if (b->graph) {
-		GP_HIP(hipGraphLaunch(b->graph, b->stream));
-	} else {
-		void *kargs[] = { &b->args };
-		k_batch_reset<<<1, 1, 0, b->stream>>>(b->d_queue);
-		GP_HIP(hipLaunchKernel(b->fn, dim3(b->grid), dim3(b->block), kargs, 0, b->stream));
-	}
+	void *kargs[] = { &b->args };
+	k_batch_reset<<<1, 1, 0, b->stream>>>(b->d_queue);
+	GP_HIP(hipLaunchKernel(b->fn, dim3(b->grid), dim3(b->block), kargs, 4 * b->args.bit_words, b->stream));
 	GP_HIP(hipEventRecord(b->e1, b->stream));
 	GP_HIP(hipStreamSynchronize(b->stream));
 	GP_HIP(hipEventElapsedTime(ms, b->e0, b->e1));
@@ -370,7 +544,7 @@ int batch_create(Che *const *meshes, uint32_t nmeshes, const uint32_t *job_mesh,
 		if (rc) return rc;
 		Che &m = *t.ren;
 		m.mean_edge = m0.mean_edge;      // the same h as the mesh itself
-		if ((rc = upload_mesh(m))) return rc;
+		if ((rc = upload_mesh(m)) || (rc = link_rows(m.dev))) return rc;
 		Layout L;
 		if ((rc = build_layout(m, nullptr, m.nv, false, L, 0, 1, 0, true))) return rc;
 		if ((rc = up(t.coff, L.coff.data(), L.coff.size())) || (rc = up(t.cid, L.cid.data(), L.cid.size())) ||
@@ -378,7 +552,7 @@ int batch_create(Che *const *meshes, uint32_t nmeshes, const uint32_t *job_mesh,
 		    (rc = up(t.cgeo64, reinterpret_cast<const double4 *>(L.cgeo64.data()), L.cgeo64.size())) ||
 		    (rc = up(t.perm, order.data(), order.size())))
 			return rc;
-		bm[k] = BMesh{ m.dev->fan_off, m.dev->fan, m.dev->closed, t.coff, t.cid, t.cgeo, t.cgeo64, nullptr, t.perm,
+		bm[k] = BMesh{ m.dev->fan_off, m.dev->fan, m.dev->link8, m.dev->closed, t.coff, t.cid, t.cgeo, t.cgeo64, nullptr, t.perm,
 		               m.dev->h, m.dev->inv_h, m.nv, L.max_slots };
 		b->max_nv = std::max(b->max_nv, m.nv);
 		b->max_slots = std::max(b->max_slots, L.max_slots);
@@ -395,14 +569,15 @@ int batch_create(Che *const *meshes, uint32_t nmeshes, const uint32_t *job_mesh,
 	b->job_nv.resize(njobs);
 	std::vector<BJob> jobs(njobs);
 	unsigned long long off = 0;
+	for (uint32_t q = 0; q < njobs; q++) {   // fields in the caller's order
+		b->out_off[q] = off;
+		b->job_nv[q] = meshes[job_mesh[q]]->nv;
+		off += b->job_nv[q];
+	}
 	for (uint32_t s = 0; s < njobs; s++) {
 		const uint32_t q = order[s];
-		const uint32_t nv = meshes[job_mesh[q]]->nv;
 		b->slot_of[q] = s;
-		b->out_off[q] = off;
-		b->job_nv[q] = nv;
-		jobs[s] = BJob{ job_mesh[q], b->tabs[job_mesh[q]].inv[job_source[q]], 0, 0, off, 0 };
-		off += nv;
+		jobs[s] = BJob{ job_mesh[q], b->tabs[job_mesh[q]].inv[job_source[q]], 0, 0, b->out_off[q], 0 };
 	}
 	b->total_out = off;
 	int rc;
@@ -432,6 +607,16 @@ int batch_create(Che *const *meshes, uint32_t nmeshes, const uint32_t *job_mesh,
 	return GP_OK;
 }
 
+// The jobs' counts of the last run (lock held).
+static int batch_jobs(gp_batch *b)
+{
+	if (!b->jobs.empty()) return GP_OK;
+	std::vector<BJob> jobs(b->njobs);
+	GP_HIP(hipMemcpy(jobs.data(), b->d_jobs, sizeof(BJob) * b->njobs, hipMemcpyDeviceToHost));
+	b->jobs.swap(jobs);
+	return GP_OK;
+}
+
 int batch_run(gp_batch *b, gp_batch_stats *st)
 {
 	if (!b) return fail(GP_ERR_INVALID, "batch is null");
@@ -439,10 +624,10 @@ int batch_run(gp_batch *b, gp_batch_stats *st)
 	int rc = batch_launch(b, &ms);
 	if (rc) return rc;
 	if (st) {
-		std::vector<BJob> jobs(b->njobs);
-		GP_HIP(hipMemcpy(jobs.data(), b->d_jobs, sizeof(BJob) * b->njobs, hipMemcpyDeviceToHost));
+		std::lock_guard<std::mutex> lock(b->mu);
+		if ((rc = batch_jobs(b))) return rc;
 		unsigned long long s = 0, r = 0;
-		for (auto &j : jobs) { s += j.sweeps; r += j.relax; }
+		for (auto &j : b->jobs) { s += j.sweeps; r += j.relax; }
 		st->sweeps = s;
 		st->relaxations = r;
 		st->vertex_fields = b->total_out;
@@ -453,19 +638,46 @@ int batch_run(gp_batch *b, gp_batch_stats *st)
 	return GP_OK;
 }
 
-int batch_result(const gp_batch *b, uint32_t job, double *dist, uint32_t cap, uint32_t *sweeps)
+__global__ void k_widen(const float *in, uint32_t n, double *out)
+{
+	for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) out[q] = in[q];
+}
+
+// Fields are read back one by one, in order as a rule: the device widens a field
+// straight into pinned memory, the WIN values from there on where the last one
+// read lies just before it, and the calls that follow copy out of there (two hipMemcpy of pageable memory a field
+// before: 59 us a field of 17k doubles, 28 now, most of it the caller's fresh pages).
+constexpr uint32_t WIN = 1u << 19;
+
+int batch_result(gp_batch *b, uint32_t job, double *dist, uint32_t cap, uint32_t *sweeps)
 {
 	if (!b || !dist) return fail(GP_ERR_INVALID, "null argument");
 	if (job >= b->njobs) return fail(GP_ERR_INVALID, "batch: job %u out of range", job);
 	const uint32_t n = b->job_nv[job];
 	if (cap < n) return fail(GP_ERR_CAPACITY, "batch: result of job %u needs %u entries", job, n);
-	std::vector<float> tmp(n);
-	GP_HIP(hipMemcpy(tmp.data(), b->d_out + b->out_off[job], 4ull * n, hipMemcpyDeviceToHost));
-	for (uint32_t v = 0; v < n; v++) dist[v] = tmp[v];
+	std::lock_guard<std::mutex> lock(b->mu);
+	const unsigned long long off = b->out_off[job];
+	for (uint32_t at = 0; at < n;) {
+		const unsigned long long from = off + at;
+		if (from < b->win_at || from >= b->win_at + b->win_n) {
+			if (!b->h_win && pinned_malloc(&b->h_win, sizeof(double) * std::min<unsigned long long>(WIN, b->total_out)) != hipSuccess)
+				return fail(GP_ERR_NOMEM, "batch: pinned allocation failed");
+			const uint32_t m = (uint32_t) std::min<unsigned long long>(WIN, from == b->next_at ? b->total_out - from : n - at);
+			b->win_n = 0;
+			k_widen<<<std::min<uint32_t>(256, (m + 255) / 256), 256, 0, b->stream>>>(b->d_out + from, m, b->h_win);
+			GP_HIP(hipGetLastError());
+			GP_HIP(hipStreamSynchronize(b->stream));
+			b->win_at = from;
+			b->win_n = m;
+		}
+		const uint32_t skip = (uint32_t) (from - b->win_at), m = std::min(n - at, b->win_n - skip);
+		copy_out(dist + at, b->h_win + skip, sizeof(double) * m);
+		at += m;
+		b->next_at = off + at;
+	}
 	if (sweeps) {
-		BJob j;
-		GP_HIP(hipMemcpy(&j, b->d_jobs + b->slot_of[job], sizeof(BJob), hipMemcpyDeviceToHost));
-		*sweeps = j.sweeps;
+		if (int rc = batch_jobs(b)) return rc;
+		*sweeps = b->jobs[b->slot_of[job]].sweeps;
 	}
 	return GP_OK;
 }

@@ -612,7 +612,7 @@ int gp_batch_run(gp_batch *batch, gp_batch_stats *stats)
 
 int gp_batch_result(const gp_batch *batch, uint32_t job, double *dist, uint32_t cap, uint32_t *sweeps)
 {
-	GP_GUARD(return gp::batch_result(batch, job, dist, cap, sweeps);)
+	GP_GUARD(return gp::batch_result(const_cast<gp_batch *>(batch), job, dist, cap, sweeps);)
 }
 
 int gp_farthest_point_sampling_ptp_gpu(gp_che *mesh, uint32_t *samples, uint32_t n_init, uint32_t cap,

@@ -230,7 +230,7 @@ int fps_gpu(Che &m, uint32_t *samples, uint32_t n_init, uint32_t cap, uint64_t n
 int batch_create(Che *const *meshes, uint32_t nmeshes, const uint32_t *job_mesh, const uint32_t *job_source,
                  uint32_t njobs, double tol, uint32_t block, gp_batch **out);
 int batch_run(gp_batch *b, gp_batch_stats *st);
-int batch_result(const gp_batch *b, uint32_t job, double *dist, uint32_t cap, uint32_t *sweeps);
+int batch_result(gp_batch *b, uint32_t job, double *dist, uint32_t cap, uint32_t *sweeps);
 
 int mlp_create(uint32_t seed, gp_mlp **out);
 int mlp_params(gp_mlp *m, float *get, const float *set, uint32_t n);

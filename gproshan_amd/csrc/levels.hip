@@ -52,10 +52,6 @@ __global__ void k_lv_seed(const uint32_t *src, uint32_t first, uint32_t ns, uint
 	}
 }
 
-// First 8 link entries of each vertex in 32 bytes (NIL past the link; LONG_LINK
-// on entry 7 when the link goes on in the fan table).
-constexpr uint32_t LONG_LINK = 0x80000000u, LINK_ROW = 8;
-
 __global__ void k_link8(const uint32_t *fan_off, const uint32_t *fan, const uint8_t *closed, uint32_t nv,
                         uint32_t *link8)
 {
@@ -390,7 +386,7 @@ Levels::~Levels()
 static uint32_t fill_grid(uint32_t n) { return std::max<uint32_t>(1, std::min<uint32_t>(2048, (n + 255) / 256)); }
 
 // The mesh's link rows, built once on first use (several threads may ask).
-static int link_rows(DeviceMesh *dm)
+int link_rows(DeviceMesh *dm)
 {
 	static std::mutex mu;
 	std::lock_guard<std::mutex> lock(mu);

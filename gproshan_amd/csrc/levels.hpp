@@ -17,6 +17,11 @@
 
 namespace gp {
 
+// First 8 link entries of each vertex in 32 bytes (NIL past the link; LONG_LINK
+// on entry 7 when the link goes on in the fan table): DeviceMesh::link8.
+constexpr uint32_t LONG_LINK = 0x80000000u, LINK_ROW = 8;
+int link_rows(DeviceMesh *dm);
+
 struct LevelState;
 
 constexpr uint32_t LEVEL_KEYS = 8;   // slot classes per level in the sort key

@@ -220,7 +220,7 @@ def ptp(mesh, sources, *, precision=L.PREC_F32, result_buffer=L.RESULT_LAST_WRIT
                        coalesce=int(coalesce), tol=tol, max_sweeps=max_sweeps, grid=grid,
                        launch_mode=launch_mode, uncapped=int(uncapped), device_setup=int(device_setup),
                        fp32_geometry=int(fp32_geometry))
-    dist = np.zeros(mesh.n_vertices())
+    dist = np.empty(mesh.n_vertices())
     srt = np.zeros(mesh.n_vertices(), np.uint32)
     st = L.PtpStats()
     check(lib().gp_ptp(mesh.handle, ptr(src), len(src), C.byref(o), ptr(dist), ptr(srt), C.byref(st)))
@@ -293,12 +293,12 @@ class Plan:
         return st.as_dict()
 
     def result(self):
-        d = np.zeros(self.mesh.n_vertices())
+        d = np.empty(self.mesh.n_vertices())
         check(lib().gp_plan_result(self._h, ptr(d)))
         return d
 
     def clusters(self):
-        c = np.zeros(self.mesh.n_vertices(), np.uint32)
+        c = np.empty(self.mesh.n_vertices(), np.uint32)
         check(lib().gp_plan_clusters(self._h, ptr(c)))
         return c
 
@@ -343,7 +343,7 @@ class Batch:
 
     def result(self, job):
         n = self.meshes[int(self._jm[job])].n_vertices()
-        d = np.zeros(n)
+        d = np.empty(n)
         sw = C.c_uint32()
         check(lib().gp_batch_result(self._h, int(job), ptr(d), n, C.byref(sw)))
         return d, sw.value
