@@ -10,6 +10,7 @@
 // directly; only the few half-edges with several candidates (non-manifold
 // edges) are paired serially in the reference's order.
 #include "gp_internal.hpp"
+#include "update_step.hpp"
 
 #include <omp.h>
 
@@ -282,6 +283,7 @@ int build_layout(const Che &m, const uint32_t *order, uint32_t nr, bool f64, Lay
 			uint32_t id = a;
 			if (f64) {
 				L.cx64[at] = Edge64{ X0[0], X0[1], X0[2] };
+				if (!fan_vector(X0)) id |= F64_FLAG;
 			} else {
 				const double q0 = X0[0] * X0[0] + X0[1] * X0[1] + X0[2] * X0[2];
 				Geo64 gd{ q0 * ih2, 0, 0, 0 };

@@ -481,7 +481,8 @@ int plan_create_rings(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_
 // in the same order, contraction off, so the same bits and the same FP64
 // flags.  FP32 solves: neighbour id (F64_FLAG for a flagged corner, SLOT_WRAP
 // on slot 0 of a closed fan), FP32 and FP64 triangle geometry in units of the
-// mean edge; FP64 solves: neighbour id and the FP64 edge vector.
+// mean edge; FP64 solves: neighbour id (F64_FLAG: an edge vector out of
+// update_fan_f64's range) and the FP64 edge vector.
 template <bool F64>
 __global__ void k_master_tables(const uint32_t *fan_off, const uint32_t *fan, const uint8_t *closed, const double *gt,
                                 uint32_t nv, double ih2, uint32_t *cid, float2 *cgeo, double4 *cgeo64, Edge64 *cx64)
@@ -499,6 +500,7 @@ __global__ void k_master_tables(const uint32_t *fan_off, const uint32_t *fan, co
 			uint32_t id = a;
 			if constexpr (F64) {
 				cx64[at] = Edge64{ X0[0], X0[1], X0[2] };
+				if (!fan_vector(X0)) id |= F64_FLAG;
 			} else {
 				const double q0 = X0[0] * X0[0] + X0[1] * X0[1] + X0[2] * X0[2];
 				double4 gd = make_double4(q0 * ih2, 0, 0, 0);

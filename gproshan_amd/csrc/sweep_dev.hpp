@@ -52,13 +52,14 @@ __device__ __forceinline__ double tri_f64(const Edge64 &xa, const Edge64 &xb, do
 	return update_ref_f64_x(X0, X1, ta, tb);
 }
 
-// The same with each fan entry's |X|^2 and |X| formed once by the caller.
+// The same with each fan entry's |X|^2 and |X| formed once by the caller, for
+// edge vectors without F64_FLAG.
 __device__ __forceinline__ double tri_f64_q(const Edge64 &xa, const Edge64 &xb, double qa, double qb, double sa,
                                             double sb, double ta, double tb)
 {
 	const double X0[3] = { xa.x, xa.y, xa.z };
 	const double X1[3] = { xb.x, xb.y, xb.z };
-	return update_ref_f64_q(X0, X1, qa, qb, sa, sb, ta, tb);
+	return update_fan_f64(X0, X1, qa, qb, sa, sb, ta, tb);
 }
 
 __device__ __forceinline__ double edge_sq(const Edge64 &x)
@@ -118,6 +119,118 @@ __device__ __forceinline__ float relax_closed(const A &a, const float2 (&g)[MS],
 	return best;
 }
 
+// The same in FP64 (no edge vector flagged).
+template <uint32_t SC, uint32_t MS>
+__device__ __forceinline__ double relax_closed(const Edge64 (&g)[MS], const double (&t)[MS], double best)
+{
+	const double q_0 = edge_sq(g[0]), s_0 = fan_sqrt(q_0);
+	double q_a = q_0, s_a = s_0;
+#pragma unroll
+	for (uint32_t k = 0; k < SC; k++) {
+		const uint32_t kn = k + 1 < SC ? k + 1 : 0;
+		double q_b = q_0, s_b = s_0;
+		if (kn) {
+			q_b = edge_sq(g[kn]);
+			s_b = fan_sqrt(q_b);
+		}
+		const double p = tri_f64_q(g[k], g[kn], q_a, q_b, s_a, s_b, t[k], t[kn]);
+		if (p < best) best = p;
+		q_a = q_b;
+		s_a = s_b;
+	}
+	return best;
+}
+
+// FP64 relaxation of a lane with at most MS slots, held in registers: lowers
+// best (and sets bk) and returns true, or returns false, nothing touched, when a
+// lane of the wave has a flagged edge vector (out of update_fan_f64's range; the
+// streaming path then).
+template <uint32_t ST, bool CL, uint32_t MS, typename A, typename OD>
+__device__ __forceinline__ bool relax_fan_f64(const A &a, size_t base, uint32_t S, const OD &od, double &best, uint32_t &bk)
+{
+	const double old = best;
+	const Edge64 *geo = a.cx64;
+	uint32_t id[MS];
+	Edge64 g[MS];
+	double t[MS];
+	if constexpr (ST == 64) {
+		// All MS slot ids, then all MS edge vectors, through descriptors that
+		// end at the chunk's S rows, as in the FP32 path of relax_lane.
+		const uint32_t lane = threadIdx.x & 63u;
+		const size_t r0 = base - lane;
+		const size_t rs = ((size_t) __builtin_amdgcn_readfirstlane((uint32_t) (r0 >> 32)) << 32) |
+		                  __builtin_amdgcn_readfirstlane((uint32_t) r0);
+		const __amdgpu_buffer_rsrc_t rid = rows_rsrc(a.cid + rs, S * 64u * 4u);
+#pragma unroll
+		for (uint32_t k = 0; k < MS; k++) id[k] = (uint32_t) raw_load_i32(rid, (int) (lane * 4u + k * 256u), 0, 0);
+		const __amdgpu_buffer_rsrc_t rg = rows_rsrc(geo + rs, S * 64u * (uint32_t) sizeof(Edge64));
+#pragma unroll
+		for (uint32_t k = 0; k < MS; k++) {
+			const int o = (int) ((lane + 64u * k) * (uint32_t) sizeof(Edge64));
+			const f64x2_t xy = raw_load_f64x2(rg, o, 0, 0);
+			g[k] = Edge64{ xy.x, xy.y, raw_load_f64(rg, o + 16, 0, 0) };
+		}
+	} else {
+		// Vertex-major tables (a lane's own S): every slot id before any
+		// edge vector, slots past S rereading the lane's last row.
+		if (S == 0) return true;
+#pragma unroll
+		for (uint32_t k = 0; k < MS; k++) id[k] = a.cid[base + ST * (k < S ? k : S - 1)];
+#pragma unroll
+		for (uint32_t k = 0; k < MS; k++) g[k] = geo[base + ST * (k < S ? k : S - 1)];
+#pragma unroll
+		for (uint32_t k = 0; k < MS; k++) id[k] = k < S ? id[k] : 0u;
+	}
+	const bool wrap = (id[0] & SLOT_WRAP) != 0u;
+	uint32_t flags = 0;
+#pragma unroll
+	for (uint32_t k = 0; k < MS; k++) flags |= id[k];
+	if (__ballot((flags & F64_FLAG) != 0u) != 0) return false;
+	gather_slots(od, id, S, t);
+	// Closed fans without empty slots, all of the chunk's length: no selects.
+	if constexpr (!CL && ST == 64) {
+		if (__ballot(!wrap || (flags & SLOT_EMPTY)) == 0 && S == 6) {
+			best = relax_closed<6>(g, t, best);
+			return true;
+		}
+	}
+	// Slot k + 1 is real (else the triangle of slot k closes onto slot 0).
+	auto next_real = [&](uint32_t k) {
+		return k + 1 < MS && k + 1 < S && !(id[(k + 1) % MS] & SLOT_EMPTY);
+	};
+	// Each entry's |X|^2 and |X| once per fan (rolled from one triangle to the
+	// next; entry 0's kept for the closing triangle).
+	const double q_0 = edge_sq(g[0]), s_0 = fan_sqrt(q_0);
+	double q_a = q_0, s_a = s_0;
+#pragma unroll
+	for (uint32_t k = 0; k < MS; k++) {
+		if (k < S) {
+			const bool nr = next_real(k);
+			const bool tri = !(id[k] & SLOT_EMPTY) && (nr || wrap);
+			const double tb = nr ? t[(k + 1) % MS] : t[0];
+			const Edge64 gb = nr ? g[(k + 1) % MS] : g[0];
+			double q_n = q_0, s_n = s_0;
+			if (k + 1 < MS && k + 1 < S) {
+				q_n = edge_sq(g[(k + 1) % MS]);
+				s_n = fan_sqrt(q_n);
+			}
+			const double q_b = nr ? q_n : q_0, s_b = nr ? s_n : s_0;
+			if (tri) {
+				const double p = tri_f64_q(g[k], gb, q_a, q_b, s_a, s_b, t[k], tb);
+				if (p < best) {
+					best = p;
+					if constexpr (CL) bk = k;
+				} else if constexpr (CL) {
+					if (p == best && p < old && k < bk) bk = k;
+				}
+			}
+			q_a = q_n;
+			s_a = s_n;
+		}
+	}
+	return true;
+}
+
 template <bool F64, uint32_t ST = 64, bool PF = true, bool CL = false, uint32_t MS = MAXS, bool G64 = false,
           typename A, typename OD>
 __device__ __forceinline__ typename std::conditional<F64, double, float>::type
@@ -175,128 +288,98 @@ relax_lane(const A &a, size_t base, uint32_t S, const OD &od, typename std::cond
 			return best;
 		}
 	}
-	if (S <= MS) {
-		// Slots past S hold id 0 (no flag bits); every use of id[k] below is
-		// guarded by k < S.
-		uint32_t id[MS];
-		G g[MS];
-		T t[MS];
-		if constexpr (ST == 64) {
-			// Chunked tables: all MS slot ids, then all MS geometry rows,
-			// through descriptors that end at the chunk's S rows (a row past
-			// S reads as 0, so id[k] = 0 there, with no branch and no memory
-			// access).  The loads are straight-line and their count fixed, so
-			// the closed-fan test and the neighbour gathers wait only for the
-			// ids (loads return in order) while the geometry is arriving.
-			// Every chunked caller passes base = (first slot row) * 64 + lane
-			// and one S for the whole wave, so the descriptors are uniform.
-			const uint32_t lane = threadIdx.x & 63u;
-			const size_t r0 = base - lane;   // the chunk's first slot, the same in every lane
-			const size_t rs = ((size_t) __builtin_amdgcn_readfirstlane((uint32_t) (r0 >> 32)) << 32) |
-			                  __builtin_amdgcn_readfirstlane((uint32_t) r0);
-			const __amdgpu_buffer_rsrc_t rid = rows_rsrc(a.cid + rs, S * 64u * 4u);
+	if constexpr (F64) {
+		if (S <= MS && relax_fan_f64<ST, CL, MS>(a, base, S, od, best, bk)) {
+			if constexpr (CL) *bk_out = bk;
+			return best;
+		}
+	}
+	if (!F64 && S <= MS) {
+		if constexpr (!F64) {
+			// Slots past S hold id 0 (no flag bits); every use of id[k] below is
+			// guarded by k < S.
+			uint32_t id[MS];
+			G g[MS];
+			T t[MS];
+			if constexpr (ST == 64) {
+				// Chunked tables: all MS slot ids, then all MS geometry rows,
+				// through descriptors that end at the chunk's S rows (a row past
+				// S reads as 0, so id[k] = 0 there, with no branch and no memory
+				// access).  The loads are straight-line and their count fixed, so
+				// the closed-fan test and the neighbour gathers wait only for the
+				// ids (loads return in order) while the geometry is arriving.
+				// Every chunked caller passes base = (first slot row) * 64 + lane
+				// and one S for the whole wave, so the descriptors are uniform.
+				const uint32_t lane = threadIdx.x & 63u;
+				const size_t r0 = base - lane;   // the chunk's first slot, the same in every lane
+				const size_t rs = ((size_t) __builtin_amdgcn_readfirstlane((uint32_t) (r0 >> 32)) << 32) |
+				                  __builtin_amdgcn_readfirstlane((uint32_t) r0);
+				const __amdgpu_buffer_rsrc_t rid = rows_rsrc(a.cid + rs, S * 64u * 4u);
 #pragma unroll
-			for (uint32_t k = 0; k < MS; k++) id[k] = (uint32_t) raw_load_i32(rid, (int) (lane * 4u + k * 256u), 0, 0);
-			const __amdgpu_buffer_rsrc_t rg = rows_rsrc(geo + rs, S * 64u * (uint32_t) sizeof(G));
+				for (uint32_t k = 0; k < MS; k++) id[k] = (uint32_t) raw_load_i32(rid, (int) (lane * 4u + k * 256u), 0, 0);
+				const __amdgpu_buffer_rsrc_t rg = rows_rsrc(geo + rs, S * 64u * (uint32_t) sizeof(G));
 #pragma unroll
-			for (uint32_t k = 0; k < MS; k++) {
-				const int o = (int) ((lane + 64u * k) * (uint32_t) sizeof(G));
-				if constexpr (F64) {
-					const f64x2_t xy = raw_load_f64x2(rg, o, 0, 0);
-					g[k] = Edge64{ xy.x, xy.y, raw_load_f64(rg, o + 16, 0, 0) };
-				} else {
-					const f32x2_t v = raw_load_f32x2(rg, o, 0, 0);
+				for (uint32_t k = 0; k < MS; k++) {
+					const f32x2_t v = raw_load_f32x2(rg, (int) ((lane + 64u * k) * (uint32_t) sizeof(G)), 0, 0);
 					g[k] = make_float2(v.x, v.y);
 				}
-			}
-		} else if constexpr (F64) {
-			// Vertex-major tables (a lane's own S): every slot id before any
-			// edge vector, slots past S rereading the lane's last row.
-			if (S == 0) return best;
+			} else {
 #pragma unroll
-			for (uint32_t k = 0; k < MS; k++) id[k] = a.cid[base + ST * (k < S ? k : S - 1)];
-#pragma unroll
-			for (uint32_t k = 0; k < MS; k++) g[k] = geo[base + ST * (k < S ? k : S - 1)];
-#pragma unroll
-			for (uint32_t k = 0; k < MS; k++) id[k] = k < S ? id[k] : 0u;
-		} else {
-#pragma unroll
-			for (uint32_t k = 0; k < MS; k++) {
-				id[k] = 0;
-				if (k < S) { id[k] = a.cid[base + ST * k]; g[k] = geo[base + ST * k]; }
-			}
-		}
-		const bool wrap = (id[0] & SLOT_WRAP) != 0u;
-		// FP32 without labels, chunked tables: when every active lane holds a
-		// closed fan without empty slots or flagged triangles (the interior of
-		// a mesh), the closed-fan path for the chunk's slot count.
-		if constexpr (!F64 && !CL && ST == 64) {
-			uint32_t flags = 0;
-#pragma unroll
-			for (uint32_t k = 0; k < MS; k++) flags |= id[k];
-			const bool plain = wrap && !(flags & (SLOT_EMPTY | F64_FLAG));
-			if (__ballot(!plain) == 0 && S >= 3 && S <= 8 && S <= MS) {
-				gather_slots(od, id, S, t);
-				switch (S) {
-				case 3: return relax_closed<3>(a, g, t, best);
-				case 4: return relax_closed<4>(a, g, t, best);
-				case 5: return relax_closed<(MS >= 5 ? 5 : MS)>(a, g, t, best);
-				case 6: return relax_closed<(MS >= 6 ? 6 : MS)>(a, g, t, best);
-				case 7: return relax_closed<(MS >= 7 ? 7 : MS)>(a, g, t, best);
-				default: return relax_closed<(MS >= 8 ? 8 : MS)>(a, g, t, best);
+				for (uint32_t k = 0; k < MS; k++) {
+					id[k] = 0;
+					if (k < S) { id[k] = a.cid[base + ST * k]; g[k] = geo[base + ST * k]; }
 				}
 			}
-		}
-		// Slot k + 1 is real (else the triangle of slot k closes onto slot 0).
-		auto next_real = [&](uint32_t k) {
-			return k + 1 < MS && k + 1 < S && !(id[(k + 1) % MS] & SLOT_EMPTY);
-		};
-		// FP32 (PF): the FP64 geometry of the first flagged triangle is
-		// requested with the neighbour distances (both depend only on the slot
-		// ids), so it costs no extra memory round trip; later flagged
-		// triangles of the lane (rare) are deferred to the loop below.  PF =
-		// false (register-tight callers) defers them all.
-		uint32_t k0 = MS, kn0 = 0;
-		double4 gd0 = { 0, 0, 0, 0 };
-		double q10 = 0;
-		if constexpr (!F64 && PF) {
+			const bool wrap = (id[0] & SLOT_WRAP) != 0u;
+			// Without labels, chunked tables: when every active lane holds a
+			// closed fan without empty slots or flagged triangles (the interior of
+			// a mesh), the closed-fan path for the chunk's slot count.
+			if constexpr (!CL && ST == 64) {
+				uint32_t flags = 0;
 #pragma unroll
-			for (uint32_t k = MS; k-- > 0;)
-				if (k < S && (id[k] & F64_FLAG)) { k0 = k; kn0 = next_real(k) ? k + 1 : 0; }
-			if (k0 != MS) {
-				gd0 = a.cgeo64[base + ST * (size_t) k0];
-				q10 = a.cgeo64[base + ST * (size_t) kn0].x;
-			}
-		}
-		gather_slots(od, id, S, t);
-		T fa = (T) INFINITY, fb = (T) INFINITY;
-		// FP64: each entry's |X|^2 and |X| once per fan (rolled from one
-		// triangle to the next; entry 0's kept for the closing triangle).
-		double q_0 = 0, s_0 = 0, q_a = 0, s_a = 0;
-		if constexpr (F64) {
-			q_0 = edge_sq(g[0]);
-			s_0 = sqrt(q_0);
-			q_a = q_0;
-			s_a = s_0;
-		}
-#pragma unroll
-		for (uint32_t k = 0; k < MS; k++) {
-			if (k < S) {
-				const bool nr = next_real(k);
-				const bool tri = !(id[k] & SLOT_EMPTY) && (nr || wrap);
-				const T tb = nr ? t[(k + 1) % MS] : t[0];
-				if constexpr (F64) {
-					const G gb = nr ? g[(k + 1) % MS] : g[0];
-					double q_n = q_0, s_n = s_0;
-					if (k + 1 < MS && k + 1 < S) {
-						q_n = edge_sq(g[(k + 1) % MS]);
-						s_n = sqrt(q_n);
+				for (uint32_t k = 0; k < MS; k++) flags |= id[k];
+				const bool plain = wrap && !(flags & (SLOT_EMPTY | F64_FLAG));
+				if (__ballot(!plain) == 0 && S >= 3 && S <= 8 && S <= MS) {
+					gather_slots(od, id, S, t);
+					switch (S) {
+					case 3: return relax_closed<3>(a, g, t, best);
+					case 4: return relax_closed<4>(a, g, t, best);
+					case 5: return relax_closed<(MS >= 5 ? 5 : MS)>(a, g, t, best);
+					case 6: return relax_closed<(MS >= 6 ? 6 : MS)>(a, g, t, best);
+					case 7: return relax_closed<(MS >= 7 ? 7 : MS)>(a, g, t, best);
+					default: return relax_closed<(MS >= 8 ? 8 : MS)>(a, g, t, best);
 					}
-					const double q_b = nr ? q_n : q_0, s_b = nr ? s_n : s_0;
-					if (tri) take(tri_f64_q(g[k], gb, q_a, q_b, s_a, s_b, t[k], tb), k);
-					q_a = q_n;
-					s_a = s_n;
-				} else {
+				}
+			}
+			// Slot k + 1 is real (else the triangle of slot k closes onto slot 0).
+			auto next_real = [&](uint32_t k) {
+				return k + 1 < MS && k + 1 < S && !(id[(k + 1) % MS] & SLOT_EMPTY);
+			};
+			// FP32 (PF): the FP64 geometry of the first flagged triangle is
+			// requested with the neighbour distances (both depend only on the slot
+			// ids), so it costs no extra memory round trip; later flagged
+			// triangles of the lane (rare) are deferred to the loop below.  PF =
+			// false (register-tight callers) defers them all.
+			uint32_t k0 = MS, kn0 = 0;
+			double4 gd0 = { 0, 0, 0, 0 };
+			double q10 = 0;
+			if constexpr (PF) {
+#pragma unroll
+				for (uint32_t k = MS; k-- > 0;)
+					if (k < S && (id[k] & F64_FLAG)) { k0 = k; kn0 = next_real(k) ? k + 1 : 0; }
+				if (k0 != MS) {
+					gd0 = a.cgeo64[base + ST * (size_t) k0];
+					q10 = a.cgeo64[base + ST * (size_t) kn0].x;
+				}
+			}
+			gather_slots(od, id, S, t);
+			T fa = (T) INFINITY, fb = (T) INFINITY;
+#pragma unroll
+			for (uint32_t k = 0; k < MS; k++) {
+				if (k < S) {
+					const bool nr = next_real(k);
+					const bool tri = !(id[k] & SLOT_EMPTY) && (nr || wrap);
+					const T tb = nr ? t[(k + 1) % MS] : t[0];
 					// Straight-line per triangle: every lane evaluates the
 					// FP32 update and keeps it only for a real, unflagged
 					// triangle; flagged ones are routed to the FP64 update by
@@ -311,12 +394,9 @@ relax_lane(const A &a, size_t base, uint32_t S, const OD &od, typename std::cond
 					fmask |= (tri && fl && k != k0) ? (1u << k) : 0u;
 				}
 			}
-		}
-		if constexpr (!F64) {
-			if (k0 != MS) {
-				take((T) update_stable<double>(gd0.x, q10, gd0.y, gd0.z, gd0.w, (double) fa, (double) fb,
-				                               (double) a.h, (double) a.inv_h), k0);
-			}
+			if (k0 != MS)
+				take((T) update_stable<double>(gd0.x, q10, gd0.y, gd0.z, gd0.w, (double) fa, (double) fb, (double) a.h,
+				                               (double) a.inv_h), k0);
 		}
 	} else {
 		const uint32_t id0 = a.cid[base];

@@ -23,9 +23,7 @@ namespace gp {
 // caller, as in the reference.
 //
 // |X|^2 as the reference forms q00 and q11 (and the square under the edge
-// paths' sqrt): the same expression, so a caller holding a whole fan can form
-// it, and its square root, once per fan entry and pass them in
-// (update_ref_f64_q) with the same bits as a result.
+// paths' sqrt).
 GP_HD double ref_sq(const double X[3])
 {
 #ifdef __clang__
@@ -34,13 +32,13 @@ GP_HD double ref_sq(const double X[3])
 	return X[0] * X[0] + X[1] * X[1] + X[2] * X[2];
 }
 
-template <bool PRE>
-GP_HD double update_ref_core(const double X0[3], const double X1[3], double q00, double q11, double s0, double s1,
-                             double t0, double t1)
+GP_HD double update_ref_f64_x(const double X0[3], const double X1[3], double t0, double t1)
 {
 #ifdef __clang__
 #pragma clang fp contract(off)
 #endif
+	const double q00 = ref_sq(X0);
+	const double q11 = ref_sq(X1);
 	const double q01 = X0[0] * X1[0] + X0[1] * X1[1] + X0[2] * X1[2];
 	const double q10 = X1[0] * X0[0] + X1[1] * X0[1] + X1[2] * X0[2];
 
@@ -66,24 +64,122 @@ GP_HD double update_ref_core(const double X0[3], const double X1[3], double q00,
 	const double c1 = cond0 * Q10 + cond1 * Q11;
 
 	if (t0 == INFINITY || t1 == INFINITY || dis < 0 || c0 >= 0 || c1 >= 0) {
-		const double dp0 = t0 + (PRE ? s0 : sqrt(ref_sq(X0)));
-		const double dp1 = t1 + (PRE ? s1 : sqrt(ref_sq(X1)));
+		const double dp0 = t0 + sqrt(q00);
+		const double dp1 = t1 + sqrt(q11);
 		p = (dp1 < dp0) ? dp1 : dp0;
 	}
 	return p;
 }
 
-GP_HD double update_ref_f64_x(const double X0[3], const double X1[3], double t0, double t1)
+// Seed of a reciprocal: 24 good bits or more.
+GP_HD double rcp_seed(double x)
 {
-	return update_ref_core<false>(X0, X1, ref_sq(X0), ref_sq(X1), 0.0, 0.0, t0, t1);
+#ifdef __HIP_DEVICE_COMPILE__
+	return __builtin_amdgcn_rcp(x);
+#else
+	const double r = 1.0 / x;
+	if (!(r * 0 == 0)) return r;
+	const double c = r * 134217729.0;   // Dekker's split: the upper 26 bits
+	return c - (c - r);
+#endif
 }
 
-// The same with q00 = ref_sq(X0), q11 = ref_sq(X1), s0 = sqrt(q00) and
-// s1 = sqrt(q11) supplied by the caller.
-GP_HD double update_ref_f64_q(const double X0[3], const double X1[3], double q00, double q11, double s0, double s1,
-                              double t0, double t1)
+// Square root of a number that is 0, negative or NaN (then the result is 0, any
+// number or NaN) or in [2^-950, 2^950], correctly rounded: Goldschmidt's iteration
+// from the reciprocal root and two corrections by the exact residual (Markstein,
+// as below).  sqrt() scales its argument and sorts out special cases besides.
+GP_HD double fan_sqrt(double x)
 {
-	return update_ref_core<true>(X0, X1, q00, q11, s0, s1, t0, t1);
+	const double c = fmax(x, 0x1p-1000);   // no 0 * inf
+#ifdef __HIP_DEVICE_COMPILE__
+	const double y = __builtin_amdgcn_rsq(c);
+#else
+	const double y = rcp_seed(sqrt(c));
+#endif
+	double g = x * y, h = 0.5 * y;
+	const double r = __builtin_fma(-h, g, 0.5);
+	g = __builtin_fma(g, r, g);
+	h = __builtin_fma(h, r, h);
+	g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+	return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
+// Edge vectors that update_fan_f64 takes: not 0, every component 0 or of a
+// magnitude in [2^-100, 2^100].  The products and sums below then neither overflow
+// nor lose bits to underflow: the dot products are 0 or at least 2^-253, det 0 or
+// at least 2^-559, all below 2^410.
+constexpr double FAN_MIN = 0x1p-100, FAN_MAX = 0x1p100;
+GP_HD bool fan_component(double x) { return x == 0 || (fabs(x) >= FAN_MIN && fabs(x) <= FAN_MAX); }
+GP_HD bool fan_vector(const double X[3])
+{
+	return fan_component(X[0]) && fan_component(X[1]) && fan_component(X[2]) && (X[0] != 0 || X[1] != 0 || X[2] != 0);
+}
+
+// The value of update_ref_f64_x, bit for bit, from the squares and lengths of the
+// edges (q, and s by fan_sqrt) in 0.6 of its operations; large FP64 sweeps are
+// bound by them: 1M vertices of 16 sources 9.70 -> 8.37 ms with it and the
+// closed-fan path of the sweeps, 66k vertices' sampling 27.2 -> 25.8 ms.
+//
+// The three quotients by det share one reciprocal: seed and two Newton steps,
+// then q = n r, q + (n - det q) r, which is the correctly rounded quotient
+// (P. Markstein, Computation of elementary functions on the IBM RISC System/6000
+// processor, IBM J. Res. Dev. 34, 1990) as nothing overflows or underflows here.
+// For det = 0 all three are NaN; the reference's are not, but p is NaN either
+// way, and the edge paths are taken for the same inputs.
+//
+// Of c0 and c1 only the signs are used.  In exact arithmetic c is Q (t - p), so
+// its signs are those of A0 = q11 tp0 - q01 tp1 and A1 = q00 tp1 - q01 tp0
+// (det > 0).  The rounding of c, and of det and Q in it, comes to less than
+// 2^-46 q00 q11 / det (s1 |tp0| + s0 |tp1|) times s1 or s0 in these units (the
+// entries of Q are at most q / det, |q01| <= s0 s1; under a hundred roundings);
+// where |A| exceeds 2^-43 of that both signs are certain, else c is formed as the
+// reference forms it.
+GP_HD double update_fan_f64(const double X0[3], const double X1[3], double q00, double q11, double s0, double s1,
+                            double t0, double t1)
+{
+#ifdef __clang__
+#pragma clang fp contract(off)
+#endif
+	const double q01 = X0[0] * X1[0] + X0[1] * X1[1] + X0[2] * X1[2];   // = the reference's q10
+	const double qq = q00 * q11;
+	const double det = qq - q01 * q01;
+
+	double r = rcp_seed(det);
+	r = __builtin_fma(r, __builtin_fma(-det, r, 1.0), r);
+	r = __builtin_fma(r, __builtin_fma(-det, r, 1.0), r);
+	auto quot = [&](double n) {
+		const double q = n * r;
+		return __builtin_fma(__builtin_fma(-det, q, n), r, q);
+	};
+	const double Q00 = quot(q11);
+	const double Q01 = quot(-q01);
+	const double Q11 = quot(q00);
+
+	const double s = Q00 + Q01 + Q01 + Q11;
+	const double delta = t0 * (Q00 + Q01) + t1 * (Q01 + Q11);
+	const double dis = delta * delta - s * (t0 * t0 * Q00 + t0 * t1 * (Q01 + Q01) + t1 * t1 * Q11 - 1);
+	double p = (delta + fan_sqrt(dis)) / s;
+
+	const double tp0 = t0 - p, tp1 = t1 - p;
+	const double A0 = __builtin_fma(tp0, q11, -(tp1 * q01));
+	const double A1 = __builtin_fma(tp1, q00, -(tp0 * q01));
+	const double M = 0x1p-43 * (qq * __builtin_fma(s1, fabs(tp0), s0 * fabs(tp1)));
+	const bool certain = fabs(A0) * det > M * s1 && fabs(A1) * det > M * s0;
+	bool edge = t0 == INFINITY || t1 == INFINITY || dis < 0 || A0 > 0 || A1 > 0;
+	if (!certain && !(t0 == INFINITY || t1 == INFINITY || dis < 0)) {
+		const double n0 = tp0 * (X0[0] * Q00 + X1[0] * Q01) + tp1 * (X0[0] * Q01 + X1[0] * Q11);
+		const double n1 = tp0 * (X0[1] * Q00 + X1[1] * Q01) + tp1 * (X0[1] * Q01 + X1[1] * Q11);
+		const double n2 = tp0 * (X0[2] * Q00 + X1[2] * Q01) + tp1 * (X0[2] * Q01 + X1[2] * Q11);
+		const double cond0 = X0[0] * n0 + X0[1] * n1 + X0[2] * n2;
+		const double cond1 = X1[0] * n0 + X1[1] * n1 + X1[2] * n2;
+		edge = cond0 * Q00 + cond1 * Q01 >= 0 || cond0 * Q01 + cond1 * Q11 >= 0;
+	}
+	if (edge) {
+		const double dp0 = t0 + s0;
+		const double dp1 = t1 + s1;
+		p = (dp1 < dp0) ? dp1 : dp0;
+	}
+	return p;
 }
 
 // The same from the three positions: X0 = ga - gv, X1 = gb - gv, as the
