@@ -162,8 +162,7 @@ __global__ void k_band_levels(uint32_t *level, const double *dhat, uint32_t nv, 
 		level[v] = b;
 		m = max(m, b);
 	}
-	for (uint32_t o = 32; o > 0; o >>= 1) m = max(m, (uint32_t) __shfl_xor(m, o));
-	if ((threadIdx.x & 63u) == 0) atomicMax(bmax, m);
+	max_into(m, bmax);
 }
 
 // Drops the empty bands from limits[0 .. *nl - 1] (a level with no vertex
@@ -589,8 +588,7 @@ __global__ void k_max_level(const uint32_t *level, uint32_t n, uint32_t *out)
 	uint32_t m = 0;
 	for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
 		if (level[v] != GP_NIL) m = max(m, level[v]);
-	for (uint32_t o = 32; o > 0; o >>= 1) m = max(m, (uint32_t) __shfl_xor((int) m, (int) o));
-	if ((threadIdx.x & 63u) == 0 && m) atomicMax(out, m);
+	max_into(m, out);
 }
 
 // Rings from the caller: the ring of each vertex (NIL: in none) and the limits.
@@ -661,7 +659,7 @@ static int create_device(Che *mesh, const uint32_t *src, uint32_t ns, const gp_p
 		double *const d_dhat = dhatb.p;
 		uint32_t *const d_bmax = bmaxb.p;
 		if (dhat) GP_HIP(hipMemcpy(d_dhat, dhat, sizeof(double) * mesh->nv, hipMemcpyHostToDevice));
-		const uint32_t gb = std::max<uint32_t>(1, std::min<uint32_t>(2048, (mesh->nv + 255) / 256));
+		const uint32_t gb = std::max<uint32_t>(1, std::min<uint32_t>(512, (mesh->nv + 255) / 256));
 		if (!dhat) {
 			k_fill_u32<<<1, 64, 0, p->stream>>>(d_bmax, 1, 0);
 			k_max_level<<<gb, 256, 0, p->stream>>>(lv.level, mesh->nv, d_bmax);
