@@ -70,6 +70,7 @@ struct FArgs {
 	const uint32_t *limits;                 // rings of the current samples (device)
 	void *dist0, *dist1;                    // by position
 	double tol;
+	uint32_t grid;
 };
 
 // Sweep k of a round: the reference loop tail on the previous state, then the
@@ -133,18 +134,16 @@ __global__ __launch_bounds__(256) void k_fps_sweep(FState *st, uint32_t k4, FArg
 	const T *od = (const T *) (cur.d ? a.dist1 : a.dist0);
 	T *nd = (T *) (cur.d ? a.dist0 : a.dist1);
 	const uint32_t c0 = start >> 6, c1 = (end + 63u) >> 6;
-	const uint32_t lane = threadIdx.x & 63u;
-	// XCD-aware split: workgroups b % 8 == x take the x-th contiguous eighth
+	const uint32_t lane = threadIdx.x;
+	// XCD-aware split: workgroups (of one wave) b % 8 == x take the x-th contiguous eighth
 	// of the window's chunks.
-	const uint32_t ngrp = gridDim.x < 8u ? gridDim.x : 8u;
+	const uint32_t ngrp = min(a.grid, 8u);
 	const uint32_t x = blockIdx.x & 7u;
-	const uint32_t nbx = (gridDim.x - x + 7u) >> 3;
-	const uint32_t wpb = blockDim.x >> 6;
-	const uint32_t lw = (blockIdx.x >> 3) * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform
+	const uint32_t nw_x = (a.grid - x + 7u) >> 3;
 	const uint32_t part = (c1 - c0 + ngrp - 1) / ngrp;
 	const uint32_t lo = c0 + x * part, hi = min(c1, lo + part);
 	uint32_t bad = 0;
-	for (uint32_t c = lo + lw; c < hi; c += nbx * wpb) {
+	for (uint32_t c = lo + (blockIdx.x >> 3); c < hi; c += nw_x) {
 		const uint32_t pos = (c << 6) + lane;
 		bool lbad = false;
 		const uint32_t cb = a.coff[c], S = a.coff[c + 1] - cb;
@@ -352,6 +351,7 @@ static int fps_impl(Che &m, uint32_t *samples, uint32_t n_init, uint32_t cap, ui
 	GP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, ms8 ? k_fps_sweep<F64, 8> : k_fps_sweep<F64, MAXS>, FB, 0));
 	const uint32_t grid = std::max<uint32_t>(8, std::min<uint32_t>((uint32_t) ncu * (uint32_t) std::max(1, occ),
 	                                                               nchunks));
+	a.grid = grid;
 	constexpr uint32_t BIG = 64, SMALL = 8;
 	auto capture = [&](uint32_t count, hipGraphExec_t *out) -> int {
 		FArgs fa = a;

@@ -124,6 +124,7 @@ int ptp_gpu_noalloc(Che &mesh, const uint32_t *d_src, uint32_t ns, const uint32_
 	a.max_iter = nl << 1;                 // src/geodesics_ptp.cpp:66-67
 	a.npos = n;
 	a.k2 = 1;
+	a.grid = ds.grid;
 	a.closed = vt.closed;
 	const uint32_t ig = std::max<uint32_t>(1, std::min<uint32_t>(1024, (n + 255) / 256));
 	k_init<double><<<ig, 256, 0, stream>>>(d0, d1, n, st, nl < 3 ? 1u : 0u);

@@ -861,7 +861,7 @@ static KArgs make_args(const gp_plan *p)
 	KArgs a{};
 	a.limits = p->d_limits; a.coff = p->d_coff; a.sb = p->sb; a.cid = p->d_cid; a.cgeo = p->d_cgeo; a.cgeo64 = p->d_cgeo64;
 	a.cx64 = p->d_cx64; a.fcum = p->d_fcum; a.order = p->d_order; a.dist0 = p->d_dist0; a.dist1 = p->d_dist1;
-	a.st = p->d_state; a.trace = p->d_trace;
+	a.st = p->d_state; a.trace = p->d_trace; a.grid = p->grid;
 	a.tol = p->opts.tol; a.h = p->dm->h; a.inv_h = p->dm->inv_h;
 	a.nl = p->nl; a.max_iter = p->max_iter; a.k2 = p->opts.uncapped ? 0u : 1u;
 	a.npos = p->n;

@@ -59,6 +59,7 @@ struct KArgs {
 	uint32_t nl, max_iter;
 	uint32_t npos;             // positions of the plan (check sweeps cover [0, npos))
 	uint32_t xblk;             // log2 of the chunk blocks dealt to XCDs (0: contiguous eighths)
+	uint32_t grid;             // workgroups of SWEEP_BLOCK threads
 	uint32_t k2;               // 1: K/2 limit (the drivers); 0: the uncapped iter_error loop
 	uint32_t *cl0, *cl1;       // cluster labels (double-buffered like the distances), or null
 	const uint8_t *closed;     // vertex-major sweeps: closed-fan flags of the mesh
@@ -80,21 +81,19 @@ __device__ __forceinline__ uint32_t sweep_body(const KArgs &a, uint32_t start, u
 	using T = typename std::conditional<F64, double, float>::type;
 	if (start >= end) return 0;
 	const uint32_t c0 = start >> 6, c1 = (end + 63u) >> 6;
-	const uint32_t lane = threadIdx.x & 63u;
+	const uint32_t lane = threadIdx.x;
 	// XCD-aware split: workgroups b with b % 8 == x run on XCD x.  xblk == 0:
 	// XCD x takes the x-th contiguous eighth of the window's chunks.  xblk > 0:
 	// chunks are dealt to XCDs in blocks of 2^xblk, block q to XCD q % 8, so a
 	// chunk is relaxed on the same XCD in every sweep (its tables and its
 	// neighbours' values stay in that XCD's L2).
 	const uint32_t x = blockIdx.x & 7u;
-	const uint32_t nbx = (gridDim.x - x + 7u) >> 3;
-	const uint32_t wpb = blockDim.x >> 6;
-	// The wave's index, taken from the first lane: the same for the whole
-	// wave, and known to the compiler as such, so the chunk index, its slot
-	// rows and the slot count live in scalar registers and the per-slot tests
-	// are scalar branches instead of per-lane compares and exec masks.
-	const uint32_t lw = (blockIdx.x >> 3) * wpb + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-	const uint32_t nw_x = nbx * wpb;
+	// One wave a workgroup: the wave's index is scalar, and so are the chunk
+	// index, its slot rows and the slot count.  The grid is an argument: from the
+	// hidden ones gridDim and blockDim are two more reads in a row, behind the
+	// slot's (1,000 of a short sweep's 8,000 cycles).
+	const uint32_t nw_x = (a.grid - x + 7u) >> 3;
+	const uint32_t lw = blockIdx.x >> 3;
 	uint32_t bad = 0;
 	static_assert(!(VM && CL), "vertex-major sweeps carry no labels");
 	auto chunk = [&](uint32_t c) {
@@ -150,7 +149,7 @@ __device__ __forceinline__ uint32_t sweep_body(const KArgs &a, uint32_t start, u
 		}
 		bad += (uint32_t) __popcll(__ballot(lbad));
 	};
-	if (a.xblk && gridDim.x >= 8u) {
+	if (a.xblk && a.grid >= 8u) {
 		const uint32_t L = a.xblk, B = 1u << L;
 		const uint32_t q0 = c0 >> L, q1 = (c1 - 1) >> L;
 		const uint32_t qx = q0 + ((x + 8u - (q0 & 7u)) & 7u);     // XCD x's first block
@@ -161,7 +160,7 @@ __device__ __forceinline__ uint32_t sweep_body(const KArgs &a, uint32_t start, u
 			if (c >= c0 && c < c1) chunk(c);
 		}
 	} else {
-		const uint32_t ngrp = gridDim.x < 8u ? gridDim.x : 8u;
+		const uint32_t ngrp = min(a.grid, 8u);
 		const uint32_t len = c1 - c0;
 		const uint32_t part = (len + ngrp - 1) / ngrp;
 		const uint32_t lo = c0 + x * part;
