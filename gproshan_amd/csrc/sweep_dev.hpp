@@ -189,8 +189,8 @@ __device__ __forceinline__ bool relax_fan_f64(const A &a, size_t base, uint32_t 
 	gather_slots(od, id, S, t);
 	// Closed fans without empty slots, all of the chunk's length: no selects.
 	if constexpr (!CL && ST == 64) {
-		if (__ballot(!wrap || (flags & SLOT_EMPTY)) == 0 && S == 6) {
-			best = relax_closed<6>(g, t, best);
+		if (__ballot(!wrap || (flags & SLOT_EMPTY)) == 0 && S >= 5 && S <= 7 && S <= MS) {
+			best = S == 5 ? relax_closed<5>(g, t, best) : S == 6 ? relax_closed<6>(g, t, best) : relax_closed<7>(g, t, best);
 			return true;
 		}
 	}

@@ -185,10 +185,11 @@ constexpr uint32_t SWEEP_BLOCK = 64;
 // be preloaded into scalar registers at wave launch: the schedule slot's load
 // then does not wait for the kernel-argument segment (a.st is the same
 // pointer).
-// FP64 without labels asks for three waves a SIMD (168 registers): a 1M window is
-// 2.4 chunks a SIMD, and with two waves it would run in two rounds.
+// FP64 asks for three waves a SIMD (168 registers; with labels and long fans it
+// would spill): a 1M window is 2.4 chunks a SIMD, and with two waves it would run
+// in two rounds.
 template <bool F64, bool CL, uint32_t MS, bool G64 = false, bool VM = false>
-__global__ __launch_bounds__(256, F64 && !CL ? 3 : 1) void k_sweep(PState *st, uint32_t k4, KArgs a)
+__global__ __launch_bounds__(256, F64 && (!CL || MS <= 8) ? 3 : 1) void k_sweep(PState *st, uint32_t k4, KArgs a)
 {
 	using T = typename std::conditional<F64, double, float>::type;
 	if (k4 >= 4u) {

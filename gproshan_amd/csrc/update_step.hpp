@@ -115,17 +115,30 @@ GP_HD bool fan_vector(const double X[3])
 	return fan_component(X[0]) && fan_component(X[1]) && fan_component(X[2]) && (X[0] != 0 || X[1] != 0 || X[2] != 0);
 }
 
+GP_HD double fan_rcp(double x)
+{
+	double r = rcp_seed(x);
+	r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+	return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+}
+GP_HD double fan_quot(double n, double x, double r)
+{
+	const double q = n * r;
+	return __builtin_fma(__builtin_fma(-x, q, n), r, q);
+}
+
 // The value of update_ref_f64_x, bit for bit, from the squares and lengths of the
 // edges (q, and s by fan_sqrt) in 0.6 of its operations; large FP64 sweeps are
-// bound by them: 1M vertices of 16 sources 9.70 -> 8.37 ms with it and the
+// bound by them: 1M vertices of 16 sources 9.70 -> 8.2 ms with it and the
 // closed-fan path of the sweeps, 66k vertices' sampling 27.2 -> 25.8 ms.
 //
-// The three quotients by det share one reciprocal: seed and two Newton steps,
-// then q = n r, q + (n - det q) r, which is the correctly rounded quotient
-// (P. Markstein, Computation of elementary functions on the IBM RISC System/6000
-// processor, IBM J. Res. Dev. 34, 1990) as nothing overflows or underflows here.
-// For det = 0 all three are NaN; the reference's are not, but p is NaN either
-// way, and the edge paths are taken for the same inputs.
+// The three quotients by det share one reciprocal, and the one by s is made alike:
+// seed and two Newton steps, then q = n r, q + (n - det q) r, which is the correctly
+// rounded quotient (P. Markstein, Computation of elementary functions on the IBM
+// RISC System/6000 processor, IBM J. Res. Dev. 34, 1990) as nothing overflows or
+// underflows here.  For det = 0 all three are NaN; the reference's are not, but p
+// is NaN either way, and the edge paths are taken for the same inputs.  For s = 0
+// p is NaN, so the signs are not certain, and p is formed again.
 //
 // Of c0 and c1 only the signs are used.  In exact arithmetic c is Q (t - p), so
 // its signs are those of A0 = q11 tp0 - q01 tp1 and A1 = q00 tp1 - q01 tp0
@@ -144,29 +157,27 @@ GP_HD double update_fan_f64(const double X0[3], const double X1[3], double q00, 
 	const double qq = q00 * q11;
 	const double det = qq - q01 * q01;
 
-	double r = rcp_seed(det);
-	r = __builtin_fma(r, __builtin_fma(-det, r, 1.0), r);
-	r = __builtin_fma(r, __builtin_fma(-det, r, 1.0), r);
-	auto quot = [&](double n) {
-		const double q = n * r;
-		return __builtin_fma(__builtin_fma(-det, q, n), r, q);
-	};
-	const double Q00 = quot(q11);
-	const double Q01 = quot(-q01);
-	const double Q11 = quot(q00);
+	const double r = fan_rcp(det);
+	const double Q00 = fan_quot(q11, det, r);
+	const double Q01 = fan_quot(-q01, det, r);
+	const double Q11 = fan_quot(q00, det, r);
 
 	const double s = Q00 + Q01 + Q01 + Q11;
 	const double delta = t0 * (Q00 + Q01) + t1 * (Q01 + Q11);
 	const double dis = delta * delta - s * (t0 * t0 * Q00 + t0 * t1 * (Q01 + Q01) + t1 * t1 * Q11 - 1);
-	double p = (delta + fan_sqrt(dis)) / s;
+	const double num = delta + fan_sqrt(dis);
+	double p = fan_quot(num, s, fan_rcp(s));
 
-	const double tp0 = t0 - p, tp1 = t1 - p;
+	double tp0 = t0 - p, tp1 = t1 - p;
 	const double A0 = __builtin_fma(tp0, q11, -(tp1 * q01));
 	const double A1 = __builtin_fma(tp1, q00, -(tp0 * q01));
 	const double M = 0x1p-43 * (qq * __builtin_fma(s1, fabs(tp0), s0 * fabs(tp1)));
 	const bool certain = fabs(A0) * det > M * s1 && fabs(A1) * det > M * s0;
 	bool edge = t0 == INFINITY || t1 == INFINITY || dis < 0 || A0 > 0 || A1 > 0;
 	if (!certain && !(t0 == INFINITY || t1 == INFINITY || dis < 0)) {
+		p = num / s;   // s == 0: not NaN
+		tp0 = t0 - p;
+		tp1 = t1 - p;
 		const double n0 = tp0 * (X0[0] * Q00 + X1[0] * Q01) + tp1 * (X0[0] * Q01 + X1[0] * Q11);
 		const double n1 = tp0 * (X0[1] * Q00 + X1[1] * Q01) + tp1 * (X0[1] * Q01 + X1[1] * Q11);
 		const double n2 = tp0 * (X0[2] * Q00 + X1[2] * Q01) + tp1 * (X0[2] * Q01 + X1[2] * Q11);
