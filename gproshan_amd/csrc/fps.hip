@@ -83,7 +83,7 @@ struct FArgs {
 // read one after the other before the first row a sweep of the 66k field took
 // 6.1 us in FP64, now 5.8, and without graphs sixteen samples 26.5 -> 23.5 ms.
 template <bool F64, uint32_t MS>
-__global__ __launch_bounds__(256) void k_fps_sweep(FState *st, uint32_t k4, FArgs a)
+__global__ __launch_bounds__(256, F64 && MS <= 8 ? 3 : 1) void k_fps_sweep(FState *st, uint32_t k4, FArgs a)
 {
 	using T = typename std::conditional<F64, double, float>::type;
 	const uint32_t kp = (k4 + 3u) & 3u;
@@ -140,20 +140,52 @@ __global__ __launch_bounds__(256) void k_fps_sweep(FState *st, uint32_t k4, FArg
 	const uint32_t ngrp = min(a.grid, 8u);
 	const uint32_t x = blockIdx.x & 7u;
 	const uint32_t nw_x = (a.grid - x + 7u) >> 3;
-	const uint32_t part = (c1 - c0 + ngrp - 1) / ngrp;
-	const uint32_t lo = c0 + x * part, hi = min(c1, lo + part);
 	uint32_t bad = 0;
-	for (uint32_t c = lo + (blockIdx.x >> 3); c < hi; c += nw_x) {
-		const uint32_t pos = (c << 6) + lane;
-		bool lbad = false;
-		const uint32_t cb = a.coff[c], S = a.coff[c + 1] - cb;
-		if (pos >= start && pos < end) {
-			const T old = od[pos];
-			const T best = relax_lane<F64, 64, false, false, MS>(a.t, (size_t) cb * 64 + lane, S, od, old);
-			nd[pos] = best;
-			if (pos < cend) lbad = !(fabs((double) best - (double) old) / (double) old < a.tol);
+	auto store = [&](uint32_t pos, T old, T best) -> bool {
+		nd[pos] = best;
+		return pos < cend && !(fabs((double) best - (double) old) / (double) old < a.tol);
+	};
+	// Small windows in FP64: LPP lanes a position.
+	auto split = [&](auto lpp) {
+		constexpr uint32_t LPP = decltype(lpp)::value, N = 64 / LPP;
+		const uint32_t part = (LPP * (c1 - c0) + ngrp - 1) / ngrp;
+		const uint32_t lo = LPP * c0 + x * part, hi = min(LPP * c1, lo + part), h = lane / N;
+		for (uint32_t u = lo + (blockIdx.x >> 3); u < hi; u += nw_x) {
+			const uint32_t c = u / LPP, v = (u % LPP) * N + lane % N, pos = (c << 6) + v;
+			const uint32_t cb = a.coff[c], S = a.coff[c + 1] - cb;
+			bool lbad = false;
+			if (pos >= start && pos < end) {
+				const T old = od[pos];
+				T best = old;
+				uint32_t bk = NO_TRI;
+				const bool done = S <= MS && relax_split_f64<false, MS, LPP>(a.t, cb, S, v, h, od, best, bk);
+				if (h == 0) {
+					if (!done) best = relax_lane<true, 64, false, false, MS>(a.t, (size_t) cb * 64 + v, S, od, old);
+					lbad = store(pos, old, best);
+				}
+			}
+			bad += (uint32_t) __popcll(__ballot(lbad));
 		}
-		bad += (uint32_t) __popcll(__ballot(lbad));
+	};
+	if (F64 && c1 - c0 <= SPLIT_CHUNKS) {
+		if constexpr (F64) {
+			if (c1 - c0 <= SPLIT_CHUNKS / 2) split(std::integral_constant<uint32_t, 4>{});
+			else split(std::integral_constant<uint32_t, 2>{});
+		}
+	} else {
+		const uint32_t part = (c1 - c0 + ngrp - 1) / ngrp;
+		const uint32_t lo = c0 + x * part, hi = min(c1, lo + part);
+		for (uint32_t c = lo + (blockIdx.x >> 3); c < hi; c += nw_x) {
+			const uint32_t pos = (c << 6) + lane;
+			bool lbad = false;
+			const uint32_t cb = a.coff[c], S = a.coff[c + 1] - cb;
+			if (pos >= start && pos < end) {
+				const T old = od[pos];
+				const T best = relax_lane<F64, 64, false, false, MS>(a.t, (size_t) cb * 64 + lane, S, od, old);
+				lbad = store(pos, old, best);
+			}
+			bad += (uint32_t) __popcll(__ballot(lbad));
+		}
 	}
 	if (lane == 0 && bad) atomicAdd(&st->bad[k4], bad);
 	if (lead) {

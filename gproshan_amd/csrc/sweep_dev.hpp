@@ -231,6 +231,79 @@ __device__ __forceinline__ bool relax_fan_f64(const A &a, size_t base, uint32_t 
 	return true;
 }
 
+// FP64 relaxation of 64 / LPP positions by a wave, LPP lanes a position: lane l
+// takes one position v of the chunk and the share h of its fan's triangles; the
+// lowest result goes to all (ties to the lowest triangle, as in fan order).  The
+// triangles are half of a short sweep's chain (4,200 of 8,500 cycles) and shrink
+// with the share; in all they grow (by half with two lanes), so this is for windows
+// that leave SIMDs idle.  False, nothing touched, as relax_fan_f64.
+//
+// Up to SPLIT_CHUNKS chunks, 1,024 waves of half a chunk, one a SIMD, two lanes; up
+// to half of that four.  FP64 sweeps of 10k vertices 5.7 -> 4.9 us, 66k 6.5 -> 4.7,
+// 289k 7.5 -> 6.5; sixteen samples of the 66k mesh 24.1 -> 20.1 ms.
+constexpr uint32_t SPLIT_CHUNKS = 512;
+
+template <bool CL, uint32_t MS, uint32_t LPP, typename A, typename T>
+__device__ __forceinline__ bool relax_split_f64(const A &a, uint32_t cb, uint32_t S, uint32_t v, uint32_t h, const T *od,
+                                                double &best, uint32_t &bk)
+{
+	constexpr uint32_t H = (MS + LPP - 1) / LPP;
+	const uint32_t cbs = __builtin_amdgcn_readfirstlane(cb), k0 = h * H;
+	const __amdgpu_buffer_rsrc_t rid = rows_rsrc(a.cid + (size_t) cbs * 64, S * 64u * 4u);
+	const __amdgpu_buffer_rsrc_t rg = rows_rsrc(a.cx64 + (size_t) cbs * 64, S * 64u * (uint32_t) sizeof(Edge64));
+	// Slot 0 and the share's slots with the one after them; rows past S read as 0.
+	uint32_t id[H + 1];
+	Edge64 g[H + 1];
+	double t[H + 1];
+	const uint32_t id0 = (uint32_t) raw_load_i32(rid, (int) (v * 4u), 0, 0);
+#pragma unroll
+	for (uint32_t j = 0; j <= H; j++) id[j] = (uint32_t) raw_load_i32(rid, (int) ((k0 * 64u + v) * 4u + j * 256u), 0, 0);
+	auto edge = [&](int o) {
+		const f64x2_t xy = raw_load_f64x2(rg, o, 0, 0);
+		return Edge64{ xy.x, xy.y, raw_load_f64(rg, o + 16, 0, 0) };
+	};
+	const Edge64 g0 = edge((int) (v * 24u));
+#pragma unroll
+	for (uint32_t j = 0; j <= H; j++) g[j] = edge((int) ((k0 * 64u + v) * 24u + j * 1536u));
+	const bool wrap = (id0 & SLOT_WRAP) != 0u;
+	uint32_t flags = id0;
+#pragma unroll
+	for (uint32_t j = 0; j <= H; j++) flags |= id[j];
+	if (__ballot((flags & F64_FLAG) != 0u) != 0) return false;
+	const double t0 = od[id0 & SLOT_ID_MASK];
+#pragma unroll
+	for (uint32_t j = 0; j <= H; j++) {
+		if (k0 + j >= S) id[j] = SLOT_EMPTY;
+		t[j] = od[id[j] & SLOT_ID_MASK];
+	}
+	const double q_0 = edge_sq(g0), s_0 = fan_sqrt(q_0);
+	double q_a = edge_sq(g[0]), s_a = fan_sqrt(q_a);
+#pragma unroll
+	for (uint32_t j = 0; j < H; j++) {
+		const bool nr = !(id[j + 1] & SLOT_EMPTY);
+		const bool tri = !(id[j] & SLOT_EMPTY) && (nr || wrap);
+		const double q_n = edge_sq(g[j + 1]), s_n = fan_sqrt(q_n);
+		const double p = tri_f64_q(g[j], nr ? g[j + 1] : g0, q_a, nr ? q_n : q_0, s_a, nr ? s_n : s_0, t[j],
+		                           nr ? t[j + 1] : t0);
+		if (tri && p < best) {
+			best = p;
+			if constexpr (CL) bk = k0 + j;
+		}
+		q_a = q_n;
+		s_a = s_n;
+	}
+#pragma unroll
+	for (uint32_t o = 64 / LPP; o < 64; o <<= 1) {
+		const double ob = __shfl_xor(best, o);
+		if constexpr (CL) {
+			const uint32_t obk = __shfl_xor(bk, o);
+			if (ob < best || (ob == best && obk < bk)) bk = obk;
+		}
+		if (ob < best) best = ob;
+	}
+	return true;
+}
+
 template <bool F64, uint32_t ST = 64, bool PF = true, bool CL = false, uint32_t MS = MAXS, bool G64 = false,
           typename A, typename OD>
 __device__ __forceinline__ typename std::conditional<F64, double, float>::type

@@ -96,6 +96,30 @@ __device__ __forceinline__ uint32_t sweep_body(const KArgs &a, uint32_t start, u
 	const uint32_t lw = blockIdx.x >> 3;
 	uint32_t bad = 0;
 	static_assert(!(VM && CL), "vertex-major sweeps carry no labels");
+	// The new value (and label) of position pos, vertex v; whether it fails the
+	// ring test.
+	auto store = [&](uint32_t pos, uint32_t v, size_t base, uint32_t S, T old, T best, uint32_t bk) -> bool {
+		nd[v] = best;
+		if constexpr (CL) {
+			// The label of the nearer of the winning triangle's two other
+			// vertices (old values; ties to the first fan entry), as the
+			// reference's GPU relax does (src/cuda/geodesics_ptp.cu:266-276).
+			const uint32_t *ocl = od == (const T *) a.dist0 ? a.cl0 : a.cl1;
+			uint32_t *ncl = od == (const T *) a.dist0 ? a.cl1 : a.cl0;
+			uint32_t cl = ocl[v];
+			if (bk != NO_TRI) {
+				const uint32_t ia = a.cid[base + 64 * (size_t) bk] & SLOT_ID_MASK;
+				const uint32_t nb = bk + 1 < S ? a.cid[base + 64 * (size_t) (bk + 1)] : SLOT_EMPTY;
+				const uint32_t ib = ((nb & SLOT_EMPTY) ? a.cid[base] : nb) & SLOT_ID_MASK;
+				cl = od[ib] < od[ia] ? ocl[ib] : ocl[ia];
+			}
+			ncl[v] = cl;
+		}
+		bool lbad = false;
+		if (pos < cend) lbad = !(fabs((double) best - (double) old) / (double) old < a.tol);
+		if (CHK && best == old) lbad = false;
+		return lbad;
+	};
 	auto chunk = [&](uint32_t c) {
 		const uint32_t pos = (c << 6) + lane;
 		bool lbad = false;
@@ -128,27 +152,46 @@ __device__ __forceinline__ uint32_t sweep_body(const KArgs &a, uint32_t start, u
 			const size_t base = (size_t) cb * 64 + lane;
 			uint32_t bk = NO_TRI;
 			const T best = relax_lane<F64, 64, true, CL, MS, G64>(a, base, S, od, old, &bk);
-			nd[v] = best;
-			if constexpr (CL) {
-				// The label of the nearer of the winning triangle's two other
-				// vertices (old values; ties to the first fan entry), as the
-				// reference's GPU relax does (src/cuda/geodesics_ptp.cu:266-276).
-				const uint32_t *ocl = od == (const T *) a.dist0 ? a.cl0 : a.cl1;
-				uint32_t *ncl = od == (const T *) a.dist0 ? a.cl1 : a.cl0;
-				uint32_t cl = ocl[v];
-				if (bk != NO_TRI) {
-					const uint32_t ia = a.cid[base + 64 * (size_t) bk] & SLOT_ID_MASK;
-					const uint32_t nb = bk + 1 < S ? a.cid[base + 64 * (size_t) (bk + 1)] : SLOT_EMPTY;
-					const uint32_t ib = ((nb & SLOT_EMPTY) ? a.cid[base] : nb) & SLOT_ID_MASK;
-					cl = od[ib] < od[ia] ? ocl[ib] : ocl[ia];
-				}
-				ncl[v] = cl;
-			}
-			if (pos < cend) lbad = !(fabs((double) best - (double) old) / (double) old < a.tol);
-			if (CHK && best == old) lbad = false;
+			lbad = store(pos, v, base, S, old, best, bk);
 		}
 		bad += (uint32_t) __popcll(__ballot(lbad));
 	};
+	if constexpr (F64 && !VM) {
+		// Small windows: LPP lanes a position.
+		auto split = [&](auto lpp) {
+			constexpr uint32_t LPP = decltype(lpp)::value, N = 64 / LPP;
+			const uint32_t ngrp = min(a.grid, 8u), part = (LPP * (c1 - c0) + ngrp - 1) / ngrp;
+			const uint32_t lo = LPP * c0 + x * part, hi = min(LPP * c1, lo + part);
+			const uint32_t h = lane / N;
+			for (uint32_t u = lo + lw; u < hi; u += nw_x) {
+				const uint32_t c = u / LPP, v = (u % LPP) * N + lane % N, pos = (c << 6) + v;
+				uint32_t cb = c * a.sb, S = a.sb;
+				if (!a.sb) {
+					const uint32_t e0 = a.coff[c], e1 = a.coff[c + 1];
+					cb = e0;
+					S = e1 - e0;
+				}
+				bool lbad = false;
+				if (pos >= start && pos < end) {
+					const T old = od[pos];
+					const size_t base = (size_t) cb * 64 + v;
+					T best = old;
+					uint32_t bk = NO_TRI;
+					const bool done = S <= MS && relax_split_f64<CL, MS, LPP>(a, cb, S, v, h, od, best, bk);
+					if (h == 0) {
+						if (!done) best = relax_lane<F64, 64, true, CL, MS, G64>(a, base, S, od, old, &bk);
+						lbad = store(pos, pos, base, S, old, best, bk);
+					}
+				}
+				bad += (uint32_t) __popcll(__ballot(lbad));
+			}
+		};
+		if (!a.xblk && !a.order && c1 - c0 <= SPLIT_CHUNKS) {
+			if (c1 - c0 <= SPLIT_CHUNKS / 2) split(std::integral_constant<uint32_t, 4>{});
+			else split(std::integral_constant<uint32_t, 2>{});
+			return bad;
+		}
+	}
 	if (a.xblk && a.grid >= 8u) {
 		const uint32_t L = a.xblk, B = 1u << L;
 		const uint32_t q0 = c0 >> L, q1 = (c1 - 1) >> L;
