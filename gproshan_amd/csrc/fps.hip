@@ -145,7 +145,7 @@ __global__ __launch_bounds__(256, F64 && MS <= 8 ? 3 : 1) void k_fps_sweep(FStat
 		nd[pos] = best;
 		return pos < cend && !(fabs((double) best - (double) old) / (double) old < a.tol);
 	};
-	// Small windows in FP64: LPP lanes a position.
+	// Small windows: LPP lanes a position.
 	auto split = [&](auto lpp) {
 		constexpr uint32_t LPP = decltype(lpp)::value, N = 64 / LPP;
 		const uint32_t part = (LPP * (c1 - c0) + ngrp - 1) / ngrp;
@@ -158,20 +158,22 @@ __global__ __launch_bounds__(256, F64 && MS <= 8 ? 3 : 1) void k_fps_sweep(FStat
 				const T old = od[pos];
 				T best = old;
 				uint32_t bk = NO_TRI;
-				const bool done = S <= MS && relax_split_f64<false, MS, LPP>(a.t, cb, S, v, h, od, best, bk);
+				bool done = S <= MS;
+				if (done) {
+					if constexpr (F64) done = relax_split_f64<false, MS, LPP>(a.t, cb, S, v, h, od, best, bk);
+					else done = relax_split_f32<false, MS, LPP>(a.t, cb, S, v, h, od, best, bk);
+				}
 				if (h == 0) {
-					if (!done) best = relax_lane<true, 64, false, false, MS>(a.t, (size_t) cb * 64 + v, S, od, old);
+					if (!done) best = relax_lane<F64, 64, false, false, MS>(a.t, (size_t) cb * 64 + v, S, od, old);
 					lbad = store(pos, old, best);
 				}
 			}
 			bad += (uint32_t) __popcll(__ballot(lbad));
 		}
 	};
-	if (F64 && c1 - c0 <= SPLIT_CHUNKS) {
-		if constexpr (F64) {
-			if (c1 - c0 <= SPLIT_CHUNKS / 2) split(std::integral_constant<uint32_t, 4>{});
-			else split(std::integral_constant<uint32_t, 2>{});
-		}
+	if (c1 - c0 <= SPLIT_CHUNKS) {
+		if (c1 - c0 <= SPLIT_CHUNKS / 2) split(std::integral_constant<uint32_t, 4>{});
+		else split(std::integral_constant<uint32_t, 2>{});
 	} else {
 		const uint32_t part = (c1 - c0 + ngrp - 1) / ngrp;
 		const uint32_t lo = c0 + x * part, hi = min(c1, lo + part);

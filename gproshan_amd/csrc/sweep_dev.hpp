@@ -231,6 +231,21 @@ __device__ __forceinline__ bool relax_fan_f64(const A &a, size_t base, uint32_t 
 	return true;
 }
 
+// The lowest of a position's LPP lanes (64 / LPP apart), ties to the lowest triangle.
+template <bool CL, uint32_t LPP, typename T>
+__device__ __forceinline__ void lowest(T &best, uint32_t &bk)
+{
+#pragma unroll
+	for (uint32_t o = 64 / LPP; o < 64; o <<= 1) {
+		const T ob = __shfl_xor(best, (int) o);
+		if constexpr (CL) {
+			const uint32_t obk = __shfl_xor(bk, (int) o);
+			if (ob < best || (ob == best && obk < bk)) bk = obk;
+		}
+		if (ob < best) best = ob;
+	}
+}
+
 // FP64 relaxation of 64 / LPP positions by a wave, LPP lanes a position: lane l
 // takes one position v of the chunk and the share h of its fan's triangles; the
 // lowest result goes to all (ties to the lowest triangle, as in fan order).  The
@@ -292,15 +307,51 @@ __device__ __forceinline__ bool relax_split_f64(const A &a, uint32_t cb, uint32_
 		q_a = q_n;
 		s_a = s_n;
 	}
+	lowest<CL, LPP>(best, bk);
+	return true;
+}
+
+// The same in FP32; a flagged triangle takes its FP64 update in place.
+template <bool CL, uint32_t MS, uint32_t LPP, typename A, typename T>
+__device__ __forceinline__ bool relax_split_f32(const A &a, uint32_t cb, uint32_t S, uint32_t v, uint32_t h, const T *od,
+                                                float &best, uint32_t &bk)
+{
+	constexpr uint32_t H = (MS + LPP - 1) / LPP;
+	const uint32_t cbs = __builtin_amdgcn_readfirstlane(cb), k0 = h * H;
+	const __amdgpu_buffer_rsrc_t rid = rows_rsrc(a.cid + (size_t) cbs * 64, S * 64u * 4u);
+	const __amdgpu_buffer_rsrc_t rg = rows_rsrc(a.cgeo + (size_t) cbs * 64, S * 64u * (uint32_t) sizeof(float2));
+	uint32_t id[H + 1];
+	f32x2_t g[H + 1];
+	float t[H + 1];
+	const uint32_t id0 = (uint32_t) raw_load_i32(rid, (int) (v * 4u), 0, 0);
 #pragma unroll
-	for (uint32_t o = 64 / LPP; o < 64; o <<= 1) {
-		const double ob = __shfl_xor(best, o);
-		if constexpr (CL) {
-			const uint32_t obk = __shfl_xor(bk, o);
-			if (ob < best || (ob == best && obk < bk)) bk = obk;
-		}
-		if (ob < best) best = ob;
+	for (uint32_t j = 0; j <= H; j++) id[j] = (uint32_t) raw_load_i32(rid, (int) ((k0 * 64u + v) * 4u + j * 256u), 0, 0);
+	const f32x2_t g0 = raw_load_f32x2(rg, (int) (v * 8u), 0, 0);
+#pragma unroll
+	for (uint32_t j = 0; j <= H; j++) g[j] = raw_load_f32x2(rg, (int) ((k0 * 64u + v) * 8u + j * 512u), 0, 0);
+	const bool wrap = (id0 & SLOT_WRAP) != 0u;
+	const float t0 = od[id0 & SLOT_ID_MASK];
+#pragma unroll
+	for (uint32_t j = 0; j <= H; j++) {
+		if (k0 + j >= S) id[j] = SLOT_EMPTY;
+		t[j] = od[id[j] & SLOT_ID_MASK];
 	}
+#pragma unroll
+	for (uint32_t j = 0; j < H; j++) {
+		const bool nr = !(id[j + 1] & SLOT_EMPTY);
+		const bool tri = !(id[j] & SLOT_EMPTY) && (nr || wrap);
+		const float tb = nr ? t[j + 1] : t0;
+		float p = update_stable_q(g[j].x, nr ? g[j + 1].x : g0.x, g[j].y, t[j], tb, a.h, a.inv_h);
+		if (tri && (id[j] & F64_FLAG)) {
+			const size_t row = (size_t) cbs * 64 + v, at = row + 64 * (size_t) (k0 + j);
+			p = tri_flagged(a, at, nr ? at + 64 : row, t[j], tb);
+		}
+		if (tri && p < best) {
+			best = p;
+			if constexpr (CL) bk = k0 + j;
+		}
+	}
+	lowest<CL, LPP>(best, bk);
 	return true;
 }
 

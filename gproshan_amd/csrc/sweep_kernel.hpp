@@ -156,7 +156,7 @@ __device__ __forceinline__ uint32_t sweep_body(const KArgs &a, uint32_t start, u
 		}
 		bad += (uint32_t) __popcll(__ballot(lbad));
 	};
-	if constexpr (F64 && !VM) {
+	if constexpr (!VM && !G64) {
 		// Small windows: LPP lanes a position.
 		auto split = [&](auto lpp) {
 			constexpr uint32_t LPP = decltype(lpp)::value, N = 64 / LPP;
@@ -177,7 +177,11 @@ __device__ __forceinline__ uint32_t sweep_body(const KArgs &a, uint32_t start, u
 					const size_t base = (size_t) cb * 64 + v;
 					T best = old;
 					uint32_t bk = NO_TRI;
-					const bool done = S <= MS && relax_split_f64<CL, MS, LPP>(a, cb, S, v, h, od, best, bk);
+					bool done = S <= MS;
+					if (done) {
+						if constexpr (F64) done = relax_split_f64<CL, MS, LPP>(a, cb, S, v, h, od, best, bk);
+						else done = relax_split_f32<CL, MS, LPP>(a, cb, S, v, h, od, best, bk);
+					}
 					if (h == 0) {
 						if (!done) best = relax_lane<F64, 64, true, CL, MS, G64>(a, base, S, od, old, &bk);
 						lbad = store(pos, pos, base, S, old, best, bk);
