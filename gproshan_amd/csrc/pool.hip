@@ -165,7 +165,10 @@ hipError_t pinned_malloc_bytes(void **p, size_t bytes)
 		}
 	}
 	const hipError_t e = hipHostMalloc(p, bytes);
-	if (e != hipSuccess) return e;
+	if (e != hipSuccess) {
+		(void) hipGetLastError();
+		return e;
+	}
 	std::lock_guard<std::mutex> lock(l.mu);
 	l.used_pinned[*p] = bytes;
 	return hipSuccess;

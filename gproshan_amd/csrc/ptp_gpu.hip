@@ -800,8 +800,9 @@ static int result_out(hipStream_t stream, const T *buf, const uint32_t *inv, uin
 {
 	constexpr uint32_t PIECE = 1u << 18, ROUND = 8;   // values of a piece, pieces in flight
 	O *stage = nullptr;
-	const size_t staged = std::min<size_t>(n, (size_t) PIECE * ROUND);
-	if (pinned_malloc(&stage, sizeof(O) * staged) != hipSuccess) return fail(GP_ERR_NOMEM, "result: pinned allocation failed");
+	uint32_t pieces = ROUND;                          // fewer where so much can't be pinned
+	while (pinned_malloc(&stage, sizeof(O) * std::min<size_t>(n, (size_t) PIECE * pieces)) != hipSuccess)
+		if ((pieces /= 2) == 0) return fail(GP_ERR_NOMEM, "result: pinned allocation failed");
 	hipEvent_t ev[ROUND] = {};
 	struct Back {
 		O *s;
@@ -815,8 +816,8 @@ static int result_out(hipStream_t stream, const T *buf, const uint32_t *inv, uin
 				if (e) (void) hipEventDestroy(e);
 		}
 	} back{ stage, ev, stream };
-	for (uint32_t r0 = 0; r0 < n; r0 += PIECE * ROUND) {
-		const uint32_t rn = std::min(n - r0, PIECE * ROUND), np = (rn + PIECE - 1) / PIECE;
+	for (uint32_t r0 = 0; r0 < n; r0 += PIECE * pieces) {
+		const uint32_t rn = std::min(n - r0, PIECE * pieces), np = (rn + PIECE - 1) / PIECE;
 		for (uint32_t q = 0; q < np; q++) {
 			const uint32_t at = q * PIECE, m = std::min(rn - at, PIECE);
 			k_result<<<std::min<uint32_t>(256, (m + 255) / 256), 256, 0, stream>>>(buf, inv, r0 + at, m, none, stage + at);
