@@ -172,7 +172,8 @@ __global__ __launch_bounds__(256, F64 && MS <= 8 ? 3 : 1) void k_fps_sweep(FStat
 		}
 	};
 	if (c1 - c0 <= split_chunks<F64>(2)) {
-		if (c1 - c0 <= split_chunks<F64>(4)) split(std::integral_constant<uint32_t, 4>{});
+		if (c1 - c0 <= split_chunks<F64>(8)) split(std::integral_constant<uint32_t, 8>{});
+		else if (c1 - c0 <= split_chunks<F64>(4)) split(std::integral_constant<uint32_t, 4>{});
 		else split(std::integral_constant<uint32_t, 2>{});
 	} else {
 		const uint32_t part = (c1 - c0 + ngrp - 1) / ngrp;

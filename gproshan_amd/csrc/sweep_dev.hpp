@@ -253,18 +253,19 @@ __device__ __forceinline__ void lowest(T &best, uint32_t &bk)
 // with the share; in all they grow (by half with two lanes), so this is for windows
 // that leave SIMDs idle.  False, nothing touched, as relax_fan_f64.
 //
-// split_chunks: up to how many chunks a window is split two or four ways.  FP64 is
-// bound by the vector units as soon as each SIMD has a wave: 1,024 waves either way
+// split_chunks: up to how many chunks a window is split two, four or eight ways.
+// FP64 is bound by the vector units as soon as each SIMD has a wave: 1,024 waves
 // (66k vertices 6.5 -> 4.7 us a sweep, 10k 5.7 -> 4.9, 289k 7.5 -> 6.5; sixteen
 // samples of the 66k mesh 24.1 -> 20.1 ms; twice as far changes nothing).  FP32 waves
 // wait for memory most of the time, and four a SIMD in halves (4,096 waves, all at
 // once) or two in quarters still gain: 66k 5.3 -> 4.5 us, 289k 5.6 -> 4.9, 1M
 // 6.5 -> 6.25; with 512 and 256 chunks 289k takes 5.2 and 1M 6.4, without a limit
-// 1M takes 6.4 and its 16-source windows 8.1 instead of 7.5.
+// 1M takes 6.4 and its 16-source windows 8.1 instead of 7.5.  Eight lanes instead of
+// four up to 128 chunks: whole calls on 3k-40k vertices 1.02-1.10x.
 template <bool F64>
 __device__ constexpr uint32_t split_chunks(uint32_t lanes)
 {
-	return F64 ? 1024 / lanes : lanes == 2 ? 2048 : 512;
+	return F64 ? 1024 / lanes : lanes == 2 ? 2048 : lanes == 4 ? 512 : 128;
 }
 
 template <bool CL, uint32_t MS, uint32_t LPP, typename A, typename T>

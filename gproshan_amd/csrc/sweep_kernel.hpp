@@ -191,7 +191,8 @@ __device__ __forceinline__ uint32_t sweep_body(const KArgs &a, uint32_t start, u
 			}
 		};
 		if (!a.xblk && !a.order && c1 - c0 <= split_chunks<F64>(2)) {
-			if (c1 - c0 <= split_chunks<F64>(4)) split(std::integral_constant<uint32_t, 4>{});
+			if (c1 - c0 <= split_chunks<F64>(8)) split(std::integral_constant<uint32_t, 8>{});
+			else if (c1 - c0 <= split_chunks<F64>(4)) split(std::integral_constant<uint32_t, 4>{});
 			else split(std::integral_constant<uint32_t, 2>{});
 			return bad;
 		}
