@@ -645,17 +645,43 @@ __global__ void k_gather_tables(const uint32_t *sorted, const uint32_t *inv, con
 			const uint32_t nf = m.coff[v + 1] - mb;
 			n = (nf && m.closed[v]) ? nf - 1 : nf;
 		}
-		for (uint32_t k = 0; k < Sc; k++) {
-			const size_t at = base + 64 * (size_t) k;
-			const bool real = k < n;
-			const uint32_t id = real ? m.cid[mb + k] : 0u;
-			cid[at] = real ? (inv[id & SLOT_ID_MASK] | (id & ~SLOT_ID_MASK)) : (p | SLOT_EMPTY);
-			if constexpr (F64) {
-				cx64[at] = real ? m.cx64[mb + k] : Edge64{ 0, 0, 0 };
-			} else {
-				cgeo[at] = real ? m.cgeo[mb + k] : make_float2(0.f, 0.f);
-				if constexpr (MIDX) midx[at] = real ? mb + k : 0u;
-				else cgeo64[at] = real ? m.cgeo64[mb + k] : make_double4(0, 0, 0, 0);
+		// Four slots at a time: their ids, then the positions and the geometry
+		// they lead to, in flight together: 1M vertices in FP32 436 -> 267 us,
+		// in FP64 272 -> 175, 201k in FP32 79 -> 50.
+		for (uint32_t k0 = 0; k0 < Sc; k0 += 4) {
+			uint32_t from[4], id[4], to[4];
+			Edge64 x[4];
+			float2 g[4];
+			double4 g64[4];
+#pragma unroll
+			for (uint32_t k = 0; k < 4; k++) {
+				from[k] = k0 + k < n ? mb + k0 + k : 0u;
+				id[k] = m.cid[from[k]];
+				if (k0 + k >= n) id[k] = 0;
+			}
+#pragma unroll
+			for (uint32_t k = 0; k < 4; k++) {
+				to[k] = inv[id[k] & SLOT_ID_MASK];
+				if constexpr (F64) {
+					x[k] = m.cx64[from[k]];
+				} else {
+					g[k] = m.cgeo[from[k]];
+					if constexpr (!MIDX) g64[k] = m.cgeo64[from[k]];
+				}
+			}
+#pragma unroll
+			for (uint32_t k = 0; k < 4; k++) {
+				if (k0 + k >= Sc) break;
+				const size_t at = base + 64 * (size_t) (k0 + k);
+				const bool real = k0 + k < n;
+				cid[at] = real ? to[k] | (id[k] & ~SLOT_ID_MASK) : p | SLOT_EMPTY;
+				if constexpr (F64) {
+					cx64[at] = real ? x[k] : Edge64{ 0, 0, 0 };
+				} else {
+					cgeo[at] = real ? g[k] : make_float2(0.f, 0.f);
+					if constexpr (MIDX) midx[at] = real ? from[k] : 0u;
+					else cgeo64[at] = real ? g64[k] : make_double4(0, 0, 0, 0);
+				}
 			}
 		}
 	}
