@@ -10,9 +10,11 @@
 // values are contiguous, so each fragment is one 16-byte load; the layer
 // outputs are written back to LDS in the layout the next GEMM reads.
 //
-// Training is deterministic: each workgroup writes its gradient partial sums
-// (no float atomics) and one kernel reduces them and applies Adam to the FP32
-// master weights, then refreshes the BF16 copies.
+// Training: each workgroup writes one row of gradient partial sums; one kernel
+// adds the rows in order and applies Adam to the FP32 master weights, then
+// refreshes the BF16 copies.  Inside a workgroup the four waves' sums meet in LDS
+// float atomics, in the order the waves arrive in, so two runs differ in last
+// bits (k_mlp_grad).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -155,21 +157,18 @@ __global__ __launch_bounds__(256) void k_mlp_forward(const __bf16 *X, uint32_t n
 // per-workgroup partial sums partial[blockIdx][NPARAM]; loss partial sums in
 // lpart[blockIdx].  scale = 2 / (number of samples of the whole batch).
 //
-// Each of the four waves runs forward and backward of its own 32 samples and
-// leaves the operands of the weight gradients (h1^T, dh2^T, dh1^T, x^T) in LDS;
-// then wave w computes rows [16 w, 16 w + 16) of dW2 and dW1 over the samples
-// of all four waves, one accumulator per sample wave, added in wave order at
-// the end.  So the gradients leave the registers once, straight to the partial
-// row, with no reduction between waves: a step is bound by its latency (weights
-// in, one pass over 128 samples, 25 KB out), not by the matrix cores.  With each
-// wave holding all 96 gradient tiles and adding them to a shared copy by LDS
-// float atomics, a 16,384-sample batch (128 workgroups) took 57.5 us; 17.2 us so.
-constexpr uint32_t GW = 4;   // waves of a workgroup, 32 samples each
-
-__global__ __launch_bounds__(64 * GW) void k_mlp_grad(const __bf16 *X, const float *tgt, const uint32_t *idx,
-                                                      uint32_t n, float scale, const float *w, const __bf16 *w1,
-                                                      const __bf16 *w2, const __bf16 *w2t, float *partial,
-                                                      float *lpart)
+// Each wave keeps the gradient tiles of its own samples in registers, and the four
+// waves add theirs to one copy in LDS by float atomics: 51.4 us for 16,384
+// samples, most of it those atomics.  Waves that split the weight matrices by rows
+// and add the four waves' sums in a fixed order take 17.2 us, but training
+// magnifies last bits (an update now and then moves a weight over a BF16 rounding):
+// parameters and loss of 64 steps behind 64 others were up to 4.5e-5 from this
+// kernel's.  So the sums stay as they are.  They take the waves in the order of their
+// arrival, and two runs of this kernel differ too: over 30 seeds by 6e-6 at the most
+// after 64 steps, after 128 by more than 2e-5 in a quarter of them.
+__global__ __launch_bounds__(256) void k_mlp_grad(const __bf16 *X, const float *tgt, const uint32_t *idx, uint32_t n,
+                                                  float scale, const float *w, const __bf16 *w1, const __bf16 *w2,
+                                                  const __bf16 *w2t, float *partial, float *lpart)
 {
 	__shared__ WShared s;
 	struct WaveBuf {
@@ -180,29 +179,25 @@ __global__ __launch_bounds__(64 * GW) void k_mlp_grad(const __bf16 *X, const flo
 		__bf16 dh1t[HD * 32];  // [in][sample]
 		__bf16 xt[KP * 32];    // [feature][sample]
 	};
-	__shared__ __align__(16) WaveBuf wb[GW];
-	__shared__ float vred[3][GW][HD / 16][64];   // b1, b2, w3 sums per wave, 16-column tile and lane
-	__shared__ float sred[2][GW][4];             // b3 and loss sums per wave and lane group
+	__shared__ __align__(16) WaveBuf wb[4];
+	__shared__ float red[NPARAM];
+	__shared__ float lred;
 	stage_weights(s, w, w1, w2, w2t, true);
+	for (uint32_t q = threadIdx.x; q < NPARAM; q += blockDim.x) red[q] = 0.f;
+	if (threadIdx.x == 0) lred = 0.f;
+	__syncthreads();
 	const uint32_t l = threadIdx.x & 63u, r = l & 15u, g = l >> 4, wv = threadIdx.x >> 6;
 	WaveBuf &B = wb[wv];
-	floatx4 gw2[GW][4], gw1[GW][2];
-#pragma unroll
-	for (uint32_t a = 0; a < GW; a++) {
-#pragma unroll
+	floatx4 gw2[4][4], gw1[4][2];
+	for (uint32_t a = 0; a < 4; a++) {
 		for (uint32_t b = 0; b < 4; b++) gw2[a][b] = floatx4{ 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
 		for (uint32_t b = 0; b < 2; b++) gw1[a][b] = floatx4{ 0.f, 0.f, 0.f, 0.f };
 	}
 	float gb1[4] = { 0, 0, 0, 0 }, gb2[4] = { 0, 0, 0, 0 }, gw3[4] = { 0, 0, 0, 0 }, gb3 = 0.f, lsum = 0.f;
 	const uint32_t npair = (n + 31) / 32;
-	// Uniform over the workgroup (the barriers below): a wave past the last
-	// pair runs on zero rows with dy = 0, which adds nothing.
-	for (uint32_t p0 = blockIdx.x * GW; p0 < npair; p0 += gridDim.x * GW) {
-		const uint32_t pr = p0 + wv;
+	for (uint32_t pr = blockIdx.x * 4 + wv; pr < npair; pr += gridDim.x * 4) {
 		floatx4 a1[2][4], a2[2][4];
 		float dy[2][4];
-#pragma unroll
 		for (uint32_t half = 0; half < 2; half++) {
 			const uint32_t srow = pr * 32 + half * 16 + r;
 			bf16x8 xa;
@@ -229,7 +224,6 @@ __global__ __launch_bounds__(64 * GW) void k_mlp_grad(const __bf16 *X, const flo
 		__builtin_amdgcn_wave_barrier();
 		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 		// h1 transposed copy and dh2 = dy w3 (z2 > 0).
-#pragma unroll
 		for (uint32_t half = 0; half < 2; half++) {
 #pragma unroll
 			for (uint32_t t = 0; t < 4; t++) {
@@ -254,8 +248,14 @@ __global__ __launch_bounds__(64 * GW) void k_mlp_grad(const __bf16 *X, const flo
 		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 		__builtin_amdgcn_wave_barrier();
 		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-		// dh1 = (dh2 W2) (z1 > 0)  (M = 16 samples, N = in, K = out 64), per half.
+		// dW2[out][in] += dh2^T h1  (M = out, N = in, K = 32 samples)
 #pragma unroll
+		for (uint32_t mt = 0; mt < 4; mt++) {
+			const bf16x8 A = ld8(&B.dh2t[(mt * 16 + r) * 32 + 8 * g]);
+#pragma unroll
+			for (uint32_t nt = 0; nt < 4; nt++) gw2[mt][nt] = mfma(A, ld8(&B.h1t[(nt * 16 + r) * 32 + 8 * g]), gw2[mt][nt]);
+		}
+		// dh1 = (dh2 W2) (z1 > 0)  (M = 16 samples, N = in, K = out 64), per half.
 		for (uint32_t half = 0; half < 2; half++) {
 			const bf16x8 A0 = ld8(&B.dh2[(half * 16 + r) * HD + 8 * g]);
 			const bf16x8 A1 = ld8(&B.dh2[(half * 16 + r) * HD + 32 + 8 * g]);
@@ -273,69 +273,37 @@ __global__ __launch_bounds__(64 * GW) void k_mlp_grad(const __bf16 *X, const flo
 				}
 			}
 		}
-		__syncthreads();
-		// dW2[out][in] += dh2^T h1 and dW1[out][in] += dh1^T X for this wave's 16
-		// rows (out), K = the 32 samples of each wave in turn.
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+		// dW1[out][in] += dh1^T X  (M = out 64, N = in 32, K = 32 samples)
 #pragma unroll
-		for (uint32_t a = 0; a < GW; a++) {
-			const bf16x8 A2 = ld8(&wb[a].dh2t[(wv * 16 + r) * 32 + 8 * g]);
+		for (uint32_t mt = 0; mt < 4; mt++) {
+			const bf16x8 A = ld8(&B.dh1t[(mt * 16 + r) * 32 + 8 * g]);
 #pragma unroll
-			for (uint32_t nt = 0; nt < 4; nt++)
-				gw2[a][nt] = mfma(A2, ld8(&wb[a].h1t[(nt * 16 + r) * 32 + 8 * g]), gw2[a][nt]);
-			const bf16x8 A1 = ld8(&wb[a].dh1t[(wv * 16 + r) * 32 + 8 * g]);
-#pragma unroll
-			for (uint32_t nt = 0; nt < 2; nt++)
-				gw1[a][nt] = mfma(A1, ld8(&wb[a].xt[(nt * 16 + r) * 32 + 8 * g]), gw1[a][nt]);
+			for (uint32_t nt = 0; nt < 2; nt++) gw1[mt][nt] = mfma(A, ld8(&B.xt[(nt * 16 + r) * 32 + 8 * g]), gw1[mt][nt]);
 		}
-		__syncthreads();
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 	}
-	float *out = partial + (size_t) blockIdx.x * NPARAM;
-#pragma unroll
-	for (uint32_t q = 0; q < 4; q++) {
-		const uint32_t o = wv * 16 + 4 * g + q;
-#pragma unroll
-		for (uint32_t nt = 0; nt < 4; nt++) {
-			float t = gw2[0][nt][q];
-#pragma unroll
-			for (uint32_t a = 1; a < GW; a++) t += gw2[a][nt][q];
-			out[OFF_W2 + o * HD + nt * 16 + r] = t;
+	// Workgroup reduction in LDS, then one partial row per workgroup.
+	for (uint32_t mt = 0; mt < 4; mt++)
+		for (uint32_t q = 0; q < 4; q++) {
+			const uint32_t o = mt * 16 + 4 * g + q;
+			for (uint32_t nt = 0; nt < 4; nt++) atomicAdd(&red[OFF_W2 + o * HD + nt * 16 + r], gw2[mt][nt][q]);
+			for (uint32_t nt = 0; nt < 2; nt++) atomicAdd(&red[OFF_W1 + o * KP + nt * 16 + r], gw1[mt][nt][q]);
 		}
-#pragma unroll
-		for (uint32_t nt = 0; nt < 2; nt++) {
-			float t = gw1[0][nt][q];
-#pragma unroll
-			for (uint32_t a = 1; a < GW; a++) t += gw1[a][nt][q];
-			out[OFF_W1 + o * KP + nt * 16 + r] = t;
-		}
-	}
-	// Bias and output-layer sums: a column's lanes in wave and lane order.
-#pragma unroll
 	for (uint32_t t = 0; t < 4; t++) {
-		vred[0][wv][t][l] = gb1[t];
-		vred[1][wv][t][l] = gb2[t];
-		vred[2][wv][t][l] = gw3[t];
+		atomicAdd(&red[OFF_B1 + t * 16 + r], gb1[t]);
+		atomicAdd(&red[OFF_B2 + t * 16 + r], gb2[t]);
+		atomicAdd(&red[OFF_W3 + t * 16 + r], gw3[t]);
 	}
-	if (r == 0) {
-		sred[0][wv][g] = gb3;
-		sred[1][wv][g] = lsum;
-	}
+	if (r == 0) atomicAdd(&red[OFF_B3], gb3);
+	if (lsum != 0.f) atomicAdd(&lred, lsum);
 	__syncthreads();
-	if (threadIdx.x < 3 * HD) {
-		const uint32_t v = threadIdx.x / HD, col = threadIdx.x % HD;
-		float t = 0.f;
-#pragma unroll
-		for (uint32_t a = 0; a < GW; a++)
-#pragma unroll
-			for (uint32_t q = 0; q < 4; q++) t += vred[v][a][col >> 4][q * 16 + (col & 15u)];
-		out[(v == 0 ? OFF_B1 : v == 1 ? OFF_B2 : OFF_W3) + col] = t;
-	} else if (threadIdx.x < 3 * HD + 2) {
-		const uint32_t v = threadIdx.x - 3 * HD;
-		float t = 0.f;
-		for (uint32_t a = 0; a < GW; a++)
-			for (uint32_t q = 0; q < 4; q++) t += sred[v][a][q];
-		if (v == 0) out[OFF_B3] = t;
-		else lpart[blockIdx.x] = t;
-	}
+	for (uint32_t q = threadIdx.x; q < NPARAM; q += blockDim.x) partial[(size_t) blockIdx.x * NPARAM + q] = red[q];
+	if (threadIdx.x == 0) lpart[blockIdx.x] = lred;
 }
 
 // Sums the partials; writes the gradient (and loss) when out != null,
@@ -718,7 +686,7 @@ int mlp_train(gp_mlp *m, const float *F, const float *t, uint32_t n, uint32_t st
 	for (uint32_t q = 0; q < n; q++) perm[q] = q;
 	if (steps == 0) {
 		GP_HIP(hipMemcpy(didx.p, perm.data(), 4ull * n, hipMemcpyHostToDevice));
-		k_mlp_grad<<<grid, 64 * GW>>>((const __bf16 *) X.p, (const float *) dt.p, (const uint32_t *) didx.p, n, 2.0f / n,
+		k_mlp_grad<<<grid, 256>>>((const __bf16 *) X.p, (const float *) dt.p, (const uint32_t *) didx.p, n, 2.0f / n,
 		                          m->d.w, m->d.w1, m->d.w2, m->d.w2t, (float *) part.p, (float *) lpart.p);
 		k_mlp_adam<<<(NPARAM + ADAM_P - 1) / ADAM_P, 4 * ADAM_P>>>((const float *) part.p, grid, (const float *) lpart.p, m->d.w, m->d.m,
 		                                          m->d.v, m->d.w1, m->d.w2, m->d.w2t, 0.f, 1.f, 1.f, (float *) dg.p,
@@ -744,7 +712,7 @@ int mlp_train(gp_mlp *m, const float *F, const float *t, uint32_t n, uint32_t st
 		const float b1c = 1.f - std::pow(0.9f, (float) m->d.step), b2c = 1.f - std::pow(0.999f, (float) m->d.step);
 		const float lr_s = lr * 0.5f * (1.f + std::cos(3.14159265f * s / steps));   // cosine decay
 		const uint32_t g = std::max<uint32_t>(1, std::min<uint32_t>(grid, (bs + 127) / 128));
-		k_mlp_grad<<<g, 64 * GW>>>((const __bf16 *) X.p, (const float *) dt.p, (const uint32_t *) didx.p + cursor, bs,
+		k_mlp_grad<<<g, 256>>>((const __bf16 *) X.p, (const float *) dt.p, (const uint32_t *) didx.p + cursor, bs,
 		                       2.0f / bs, m->d.w, m->d.w1, m->d.w2, m->d.w2t, (float *) part.p, (float *) lpart.p);
 		k_mlp_adam<<<(NPARAM + ADAM_P - 1) / ADAM_P, 4 * ADAM_P>>>((const float *) part.p, g, (const float *) lpart.p, m->d.w, m->d.m,
 		                                          m->d.v, m->d.w1, m->d.w2, m->d.w2t, lr_s, b1c, b2c, nullptr,

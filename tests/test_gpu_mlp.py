@@ -1,5 +1,7 @@
 """GPU learned-band predictor: features, BF16-MFMA forward and gradients
 against the FP64 numpy oracle (oracle/mlp.py)."""
+import itertools
+
 import numpy as np
 import pytest
 
@@ -121,3 +123,23 @@ def test_gradient_does_not_depend_on_where_a_row_sits(n, copies):
     a, b = Lr.unpack(g1), Lr.unpack(g2)
     for k in a:
         assert np.linalg.norm(a[k] - b[k]) <= 1e-4 * np.linalg.norm(a[k]) + 1e-12, k
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_gradient_adds_its_waves(seed):
+    """The gradient of 128 rows, one workgroup's, is the FP32 sum of those of its
+    four waves' 32 rows in some order: of each weight's value one of the sums has
+    the bits (the waves' shares scale by a power of two, exactly)."""
+    F, t = _data(128, seed)
+    net = Lr.MLP(seed=seed)
+    part = [np.float32(0.25) * net.gradient(F[q:q + 32], t[q:q + 32])[0].astype(np.float32) for q in range(0, 128, 32)]
+    got = Lr.unpack(net.gradient(F, t)[0])
+    part = [Lr.unpack(p) for p in part]
+    for k in ("W1", "W2"):
+        hit = np.zeros(got[k].shape, bool)
+        for order in itertools.permutations(range(4)):
+            s = np.zeros(got[k].shape, np.float32)
+            for w in order:
+                s = s + part[w][k].astype(np.float32)
+            hit |= s == got[k]
+        assert hit.all(), (k, int((~hit).sum()))
