@@ -23,11 +23,12 @@ RESULT_LAST_WRITTEN, RESULT_LAST_READ = 0, 1
 SCHED_RINGS, SCHED_LEARNED_BAND, SCHED_EUCLID_BAND, SCHED_RING_BAND, SCHED_PATCHES = 0, 1, 2, 3, 4
 LAUNCH_GRAPH, LAUNCH_STREAM, LAUNCH_FLOW = 0, 1, 2
 GEO_AUTO, GEO_FP32, GEO_FP64 = 0, 1, 2
+ORDERED_LINK = 32
 
 # Every symbol include/gproshan_ptp.h declares.
 EXPORTS = [
     "gp_ptp_opts_default", "gp_last_error", "gp_device_check",
-    "gp_che_create", "gp_che_destroy", "gp_che_read", "gp_che_positions", "gp_che_sizes", "gp_che_tables", "gp_che_link", "gp_che_mean_edge",
+    "gp_che_create", "gp_che_destroy", "gp_che_read", "gp_che_positions", "gp_che_sizes", "gp_che_tables", "gp_che_link", "gp_che_mean_edge", "gp_che_max_link",
     "gp_compute_toplesets", "gp_compute_toplesets_k", "gp_compute_toplesets_gpu",
     "gp_parallel_toplesets_propagation_gpu", "gp_parallel_toplesets_propagation_coalescence_gpu",
     "gp_parallel_toplesets_propagation_gpu_noalloc",
@@ -120,6 +121,7 @@ def lib() -> C.CDLL:
     L.gp_che_tables.argtypes = [P, P, P, P]
     L.gp_che_link.argtypes = [P, u32, P, u32, C.POINTER(u32)]
     L.gp_che_mean_edge.argtypes = [P, C.POINTER(C.c_double)]
+    L.gp_che_max_link.argtypes = [P, C.POINTER(u32)]
     L.gp_compute_toplesets.argtypes = [P, P, u32, P, P, P, u32, C.POINTER(u32)]
     L.gp_compute_toplesets_gpu.argtypes = [P, P, u32, P, P, P, u32, C.POINTER(u32)]
     L.gp_compute_toplesets_k.argtypes = [P, P, u32, u32, P, P, P, u32, C.POINTER(u32)]

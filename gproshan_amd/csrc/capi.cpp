@@ -143,6 +143,15 @@ int gp_che_mean_edge(const gp_che *mesh, double *h)
 	)
 }
 
+int gp_che_max_link(const gp_che *mesh, uint32_t *n)
+{
+	GP_GUARD(
+		if (!mesh || !n) return gp::fail(GP_ERR_INVALID, "null argument");
+		*n = mesh->m.max_link;
+		return GP_OK;
+	)
+}
+
 int gp_compute_toplesets(const gp_che *mesh, const uint32_t *sources, uint32_t n_sources, uint32_t *toplesets,
                          uint32_t *sorted, uint32_t *limits, uint32_t cap_limits, uint32_t *n_limits)
 {

@@ -70,7 +70,7 @@ struct Levels {
 // (lv.sorted, lv.limits, lv.level and inv[nv], the position of each vertex in
 // lv.sorted; d_src: the sources in the caller's order).  Everything passed stays
 // unchanged and allocated until the stream has run them.
-constexpr uint32_t ORDER_MAX_LINK = 32;   // longer links: the one-workgroup BFS of rings.hip
+constexpr uint32_t ORDER_MAX_LINK = GP_ORDERED_LINK;   // longer links: the one-workgroup BFS of rings.hip
 
 struct RingOrder {
 	uint32_t *child = nullptr, *rank0 = nullptr, *work = nullptr, *out = nullptr;

@@ -121,6 +121,11 @@ class che:
         check(lib().gp_che_mean_edge(self._h, C.byref(h)))
         return h.value
 
+    def max_link(self):
+        n = C.c_uint32()
+        check(lib().gp_che_max_link(self._h, C.byref(n)))
+        return n.value
+
     def compute_toplesets(self, sources, gpu: bool = False, k: int = NIL):
         """Returns (toplesets u32[V], sorted u32[V], limits u32[R+1]); k is the
         reference's level cut (host builder only)."""
@@ -393,8 +398,11 @@ class geodesics:
             self._dist[:n] = parallel_toplesets_propagation_coalescence_cpu(mesh, src, ts)
         elif opt == self.PTP_GPU and cluster:
             # The reference's GPU drivers with their cluster output
-            # (src/geodesics.cpp:225-240).
-            ts = mesh.compute_toplesets(src, gpu=True)
+            # (src/geodesics.cpp:225-240).  Their rings come from the device where
+            # all of it orders them; past that length of a link from the host, which
+            # takes any length and is faster than one workgroup (12k vertices, a link
+            # of 60: 2.8 against 5.2 ms for the call; 120k, one of 600: 20.0 against 24.6).
+            ts = mesh.compute_toplesets(src, gpu=mesh.max_link() <= L.ORDERED_LINK)
             drv = parallel_toplesets_propagation_coalescence_gpu if len(src) == 1 else parallel_toplesets_propagation_gpu
             d, _, cl = drv(mesh, src, ts, clusters=True)
             self._sorted[:] = ts[1]

@@ -225,6 +225,13 @@ int gp_che_link(const gp_che *mesh, uint32_t v, uint32_t *he_out, uint32_t cap, 
  * the FP32 solve and of band_width. */
 int gp_che_mean_edge(const gp_che *mesh, double *h);
 
+/* Vertices of the longest link (no reference counterpart).  Up to
+ * GP_ORDERED_LINK of them the GPU's toplesets are worked out by the whole
+ * device, past that by one workgroup (at most 1,024; the host builder is then the
+ * faster one and takes any). */
+#define GP_ORDERED_LINK 32u
+int gp_che_max_link(const gp_che *mesh, uint32_t *n);
+
 /* ---- toplesets ----------------------------------------------------------- */
 
 /* che::compute_toplesets(toplesets, sorted, limits, sources) (include/che.h:107;

@@ -55,3 +55,27 @@ def test_clusters_f32_and_drivers(case, oracle):
     g = P.geodesics(C, src, P.geodesics.PTP_GPU, cluster=True)
     assert g.clusters is not None and len(g.clusters) == len(cl)
     assert int((g.clusters != cref).sum()) <= max(3, len(cl) // 10000)
+
+
+@pytest.mark.parametrize("rings,link", [(3, 32), (3, 33), (3, 64), (2, 1024), (2, 1025)])
+@pytest.mark.parametrize("src", [[5], [7, 0]])
+def test_front_end_takes_any_link(oracle, rings, link, src):
+    """Labels at and past the longest links that the device orders rings of (32,
+    by all workgroups; 1,024, by one).  The oracle's rings and labels take links to
+    64: past them its field on the host's rings, and the host-built plan's labels
+    (checked against the oracle above)."""
+    xyz, f = G.polar_disk(rings, link, 1)
+    M, C = oracle.Mesh(xyz, f), P.che(xyz, f)
+    assert C.max_link() == link
+    coal = len(src) == 1
+    variant = oracle.GPU_COAL if coal else oracle.GPU_PLAIN
+    if link <= 64:
+        dref, cref, _ = M.ptp_clusters(src, variant)
+    else:
+        dref, _ = M.ptp(src, variant, toplesets=C.compute_toplesets(src))
+        plan = P.Plan(C, src, precision=L.PREC_F64, coalesce=coal, clusters=True)
+        plan.run()
+        cref = plan.clusters()
+    g = P.geodesics(C, src, P.geodesics.PTP_GPU, cluster=True)
+    assert np.array_equal(g.dist, dref)
+    assert np.array_equal(g.clusters, cref)
