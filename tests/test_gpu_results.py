@@ -69,3 +69,35 @@ def test_memory_kept_is_bounded():
     for side in range(100, 1000, 60):
         solve(side)
     assert used() - before <= (1 << 30) + (64 << 20)
+
+
+def test_memory_kept_is_bounded_while_a_mesh_lives():
+    """One mesh's device tables keep the lists from being emptied.  Growing meshes
+    reuse hardly any block of the one before: together they drop over 2 GiB (more than 250
+    bytes a vertex in FP64), of which 1 GiB may stay.  Blocks take up to 2 MiB
+    more than asked for, at most a few dozen of them are kept: 128 MiB."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+
+    def used():
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return total.value - free.value
+
+    def solve(side):
+        xyz, f = G.height_field(side, 1)
+        P.ptp(P.che(xyz, f), [0], precision=L.PREC_F64, device_setup=True)
+
+    solve(64)
+    gone = used()
+    hold = P.che(*G.height_field(8, 1))
+    P.ptp(hold, [0], precision=L.PREC_F64, device_setup=True)
+    before = used()
+    sides = range(300, 1400, 90)
+    assert 250 * sum(s * s for s in sides) > 2 << 30
+    most = 0
+    for side in sides:
+        solve(side)
+        most = max(most, used() - before)
+    assert (1 << 29) < most <= (1 << 30) + (128 << 20), most
+    del hold
+    assert used() - gone <= 8 << 20
