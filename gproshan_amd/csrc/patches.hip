@@ -360,7 +360,7 @@ struct PatchPlan {
 		                 (void *) d_src, (void *) d_lidx, (void *) d_cgeo, (void *) d_cgeo64, (void *) d_pkey,
 		                 (void *) d_dist, (void *) d_out, (void *) d_state, (void *) d_defer })
 			(void) hipFree(p);
-		if (h_state) (void) hipHostFree(h_state);
+		pinned_free(h_state);   // behind hipFree, which waits for the device
 		if (graph) (void) hipGraphExecDestroy(graph);
 		if (e0) (void) hipEventDestroy(e0);
 		if (e1) (void) hipEventDestroy(e1);
@@ -455,7 +455,7 @@ int patch_create(Che *mesh, const uint32_t *src, uint32_t ns, const double *dhat
 	    device_malloc(&pp->d_mark, 4ull * 4 * pp->npatch) != hipSuccess || device_malloc(&pp->d_defer, pp->npatch) != hipSuccess ||
 	    device_malloc(&pp->d_trace, 32ull * trace_rows) != hipSuccess || device_malloc(&pp->d_dist, 4ull * pp->n) != hipSuccess ||
 	    device_malloc(&pp->d_out, 8ull * pp->n) != hipSuccess || device_malloc(&pp->d_state, sizeof(PatchState)) != hipSuccess ||
-	    hipHostMalloc(&pp->h_state, sizeof(PatchState)) != hipSuccess)
+	    pinned_malloc(&pp->h_state, sizeof(PatchState)) != hipSuccess)
 		return fail(GP_ERR_NOMEM, "patch plan: device allocation failed");
 	pp->max_launch = std::min(pp->max_launch, trace_rows);
 	GP_HIP(hipStreamCreateWithFlags(&pp->stream, hipStreamNonBlocking));

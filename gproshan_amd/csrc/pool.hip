@@ -164,9 +164,18 @@ hipError_t pinned_malloc_bytes(void **p, size_t bytes)
 			return hipSuccess;
 		}
 	}
-	const hipError_t e = hipHostMalloc(p, bytes);
+	hipError_t e = hipHostMalloc(p, bytes);
 	if (e != hipSuccess) {
 		(void) hipGetLastError();
+		{
+			std::lock_guard<std::mutex> lock(l.mu);
+			empty(l);
+		}
+		e = hipHostMalloc(p, bytes);
+	}
+	if (e != hipSuccess) {
+		(void) hipGetLastError();
+		*p = nullptr;
 		return e;
 	}
 	std::lock_guard<std::mutex> lock(l.mu);

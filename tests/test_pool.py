@@ -1,5 +1,6 @@
 """The memory kept between calls, its source compiled for the CPU on a stand-in of
-the HIP runtime: the bounds with a mesh alive and the order in which blocks go back."""
+the HIP runtime: the bounds with a mesh alive, the order in which blocks go back,
+and failed allocations."""
 import os
 import subprocess
 
@@ -16,7 +17,7 @@ def exe(tmp_path_factory):
     return path
 
 
-@pytest.mark.parametrize("what", ["device_bound", "pinned_bound"])
+@pytest.mark.parametrize("what", ["device_bound", "pinned_bound", "device_fails", "pinned_fails"])
 def test_pool(exe, what):
     r = subprocess.run([exe, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
