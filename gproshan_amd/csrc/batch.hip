@@ -660,8 +660,13 @@ int batch_result(gp_batch *b, uint32_t job, double *dist, uint32_t cap, uint32_t
 	for (uint32_t at = 0; at < n;) {
 		const unsigned long long from = off + at;
 		if (from < b->win_at || from >= b->win_at + b->win_n) {
-			if (!b->h_win && pinned_malloc(&b->h_win, sizeof(double) * std::min<unsigned long long>(WIN, b->total_out)) != hipSuccess)
-				return fail(GP_ERR_NOMEM, "batch: pinned allocation failed");
+			if (!b->h_win && pinned_malloc(&b->h_win, sizeof(double) * std::min<unsigned long long>(WIN, b->total_out)) != hipSuccess) {
+				// None to be had: this field by a pageable copy.
+				std::vector<float> field(n);
+				GP_HIP(hipMemcpy(field.data(), b->d_out + off, sizeof(float) * n, hipMemcpyDeviceToHost));
+				for (uint32_t v = 0; v < n; v++) dist[v] = field[v];
+				break;
+			}
 			const uint32_t m = (uint32_t) std::min<unsigned long long>(WIN, from == b->next_at ? b->total_out - from : n - at);
 			b->win_n = 0;
 			k_widen<<<std::min<uint32_t>(256, (m + 255) / 256), 256, 0, b->stream>>>(b->d_out + from, m, b->h_win);

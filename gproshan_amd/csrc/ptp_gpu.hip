@@ -128,7 +128,7 @@ __global__ void k_cl_sources(uint32_t *c0, uint32_t *c1, const uint32_t *src, ui
 
 // Values of vertices [v0, v0 + n) from the ring positions (inv; null: the buffer
 // is in the caller's numbering), `none` where unreached, straight into pinned
-// host memory.
+// host memory (or device memory on the way out, result_pageable).
 template <typename T, typename O>
 __global__ void k_result(const T *in, const uint32_t *inv, uint32_t v0, uint32_t n, O none, O *out)
 {
@@ -791,6 +791,24 @@ int plan_create_given(Che *mesh, const uint32_t *src, uint32_t ns, const uint32_
 	return plan_create_rings(mesh, src, ns, limits, nl, sorted, opts, out);
 }
 
+// The same without pinned memory: pieces by way of device memory, copied by the
+// runtime.
+template <typename T, typename O>
+static int result_pageable(hipStream_t stream, const T *buf, const uint32_t *inv, uint32_t n, O none, O *out,
+                           uint32_t piece)
+{
+	PoolBuf<O> stage(stream);
+	if (stage.alloc(sizeof(O) * std::min(n, piece)) != hipSuccess) return fail(GP_ERR_NOMEM, "result: allocation failed");
+	for (uint32_t r0 = 0; r0 < n; r0 += piece) {
+		const uint32_t m = std::min(n - r0, piece);
+		k_result<<<std::min<uint32_t>(256, (m + 255) / 256), 256, 0, stream>>>(buf, inv, r0, m, none, stage.p);
+		GP_HIP(hipGetLastError());
+		GP_HIP(hipMemcpyAsync(out + r0, stage.p, sizeof(O) * m, hipMemcpyDeviceToHost, stream));
+		GP_HIP(hipStreamSynchronize(stream));
+	}
+	return GP_OK;
+}
+
 // n values in the caller's numbering into host memory: written by the device to
 // pinned memory in pieces, each copied out by several threads while the next
 // are written.  A 1M-vertex field into a fresh array: 2.7 ms with a conversion
@@ -802,7 +820,7 @@ static int result_out(hipStream_t stream, const T *buf, const uint32_t *inv, uin
 	O *stage = nullptr;
 	uint32_t pieces = ROUND;                          // fewer where so much can't be pinned
 	while (pinned_malloc(&stage, sizeof(O) * std::min<size_t>(n, (size_t) PIECE * pieces)) != hipSuccess)
-		if ((pieces /= 2) == 0) return fail(GP_ERR_NOMEM, "result: pinned allocation failed");
+		if ((pieces /= 2) == 0) return result_pageable(stream, buf, inv, n, none, out, PIECE);
 	hipEvent_t ev[ROUND] = {};
 	struct Back {
 		O *s;
