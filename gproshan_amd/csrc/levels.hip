@@ -207,9 +207,12 @@ __global__ __launch_bounds__(LV_T) void k_lv_step(LvArgs a, uint32_t k4)
 // or reserves one global count per key present in the block.  Small meshes are
 // bound by a workgroup's own chain: with two vertices a thread, their keys held in
 // registers, and only the bins in use cleared, histogram and scatter of 66k vertices
-// take 4.9 and 5.3 us instead of 13.6 and 17.  From SORT_SMALL vertices the
-// global counts are: eight a thread.
-constexpr uint32_t SORT_SMALL = 262144;
+// take 4.9 and 5.3 us instead of 13.6 and 17.  Large ones are bound by the global
+// counts, so by the number of blocks: eight a thread.  Histogram and scatter with
+// two / eight vertices a thread, one source: 262k vertices 15.4 / 23.2 us, 410k
+// 20.7 / 25.9, 608k 21.5 / 24.6, 810k 29.9 / 27.9, 1M 31.6 / 27.6; sixteen sources:
+// 262k 14.3 / 22.2, 410k 18.8 / 22.0, 608k 26.7 / 25.2, 810k 33.4 / 26.0.
+constexpr uint32_t SORT_SMALL = 1u << 19;
 constexpr uint32_t SORT_BINS = 12288, SORT_T = 1024;
 
 // Sort key of vertex v: level * KS + slot class (KS or more slots first, then

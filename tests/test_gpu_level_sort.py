@@ -1,5 +1,5 @@
 """The counting sort by level at the edges of its blocks (2,048 vertices a
-workgroup up to 262,144 vertices, 8,192 above): the device's rings are the
+workgroup up to 524,288 vertices, 8,192 above): the device's rings are the
 host's, and a field on them has the bits of the host-built one."""
 import numpy as np
 import pytest
@@ -21,3 +21,9 @@ def test_rings_at_the_edges_of_blocks(rows, cols):
         a = P.ptp(mesh, src, precision=L.PREC_F64, device_setup=True)[0]
         b = P.ptp(mesh, src, precision=L.PREC_F64)[0]
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("rows,cols", [(512, 1024), (509, 1031), (723, 724)])
+def test_rings_about_the_larger_blocks(rows, cols):
+    """524,288 vertices, a few more, a few less."""
+    test_rings_at_the_edges_of_blocks(rows, cols)
