@@ -18,7 +18,7 @@ namespace gp {
 struct LevelState {
 	uint32_t serial[4];
 	uint32_t cnt[4];
-	uint32_t done, launches, max_level, pad;
+	uint32_t done, max_level;
 };
 
 __global__ void k_lv_zero(uint32_t *p, uint32_t n)
@@ -47,7 +47,7 @@ __global__ void k_lv_seed(const uint32_t *src, uint32_t first, uint32_t ns, uint
 			for (uint32_t q = 0; q < 4; q++) s = max(s, ls->serial[q]);
 		for (uint32_t q = 0; q < 4; q++) { ls->serial[q] = s; ls->cnt[q] = 0; }
 		ls->cnt[3] = ns - first;
-		ls->launches = ls->max_level = ls->pad = 0;
+		ls->max_level = 0;
 		ls->done = ns > first ? 0u : 1u;
 	}
 }
@@ -107,7 +107,6 @@ __global__ __launch_bounds__(LV_T) void k_lv_step(LvArgs a, uint32_t k4)
 		ls->serial[k4] = serial;
 		ls->cnt[(k4 + 1u) & 3u] = 0;
 		if (n == 0) ls->done = 1;
-		else ls->launches = ls->launches + 1;
 	}
 	// Vertex w to the next launch's frontier (every lane of the wave calls).
 	auto queue_next = [&](bool want, uint32_t w) {
