@@ -1,11 +1,14 @@
 // Batched PTP: many (mesh, source) fields of uneven size in one persistent
-// launch behind the reset of its queue.
+// launch behind the reset of its queue: two launches on the stream, for which a
+// graph has nothing to save (a launch runs for milliseconds; 1,024 fields 27 ms).
 //
 // Each 1024-thread workgroup repeatedly takes the next job from an atomic
 // queue (jobs sorted by decreasing cost V^1.5, so the grid drains evenly), and
-// runs it entirely by itself: the ring build (the same BFS as the toplesets
-// kernel), then the reference window schedule (K/2 band limit, PTP_TOL test,
-// 2*|limits| cap, last-written buffer) with __syncthreads as the only barrier,
+// runs it entirely by itself: the ring build (bfs_bits, its visited bits and
+// frontier in LDS, with barriers that wait for LDS only; meshes of more than
+// 262,144 vertices take the ordered BFS, bfs_block), then the reference window
+// schedule (K/2 band limit, PTP_TOL test, 2*|limits| cap, last-written buffer)
+// with one __syncthreads a sweep as the only barrier,
 // on the rings of the reference's non-coalesced driver
 // (src/cuda/geodesics_ptp.cu:174-299).  Each mesh is stored vertex-major (a
 // vertex's slots are contiguous) in Morton order; after its BFS the workgroup
@@ -232,6 +235,11 @@ __device__ __forceinline__ uint32_t bfs_bits(const BMesh &M, uint32_t src, uint3
 // (the units are busy 46 % of the time), a chain that four waves a SIMD cover in
 // part.  Two fields a CU of 512 threads take longer (38 ms) as they need twice
 // the cache, and asking for a chunk's rows one chunk ahead does too (29 ms).
+//
+// Four waves a SIMD is the most that is asked for.  A build of this kernel forced to
+// eight (64 registers, 304 bytes of spills a lane) ended in a GPU memory fault with
+// 1,024 threads a field; every index is bounded alike in both builds and no cause was
+// found, so it was not run again.
 constexpr uint32_t BL = 1024;   // ring limits kept in LDS
 
 template <uint32_t NT, uint32_t MS>

@@ -36,8 +36,8 @@ struct DeviceMesh {
 // Uploads the fan tables and FP64 positions of m once (m.dev caches them).
 int upload_mesh(Che &m);
 
-// Replayed launch sequences (sweeps, patch launches, the batch) run from
-// hipGraphs unless the environment sets
+// Replayed launch sequences (FP32 sweeps from a plan's second run on, FP32
+// sampling sweeps, patch launches) run from hipGraphs unless the environment sets
 // GPROSHAN_AMD_GRAPHS=0: then the same kernels are launched one by one on the
 // stream, with the same results (a profiler that cannot follow graph replays
 // traces these).

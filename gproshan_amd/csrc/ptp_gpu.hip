@@ -9,11 +9,12 @@
 //
 // The reference launches a relax kernel, a relative-error kernel and a Thrust
 // count per sweep with three host synchronisations.  Here the schedule lives
-// in device memory: a sweep kernel relaxes the window it reads from there and
-// counts non-converged ring-i vertices (wave reductions, one atomic per wave
-// with a non-zero count), and a one-thread kernel advances the schedule.  The
-// pairs are built once into a hipGraph and replayed until the device sets
-// its done flag; the host polls that flag once per replay.  (A persistent
+// in device memory: a sweep kernel advances it by the outcome of the sweep
+// before, relaxes the window it reads from there and counts non-converged ring-i
+// vertices (wave reductions, one atomic per wave with a non-zero count).  Sweeps
+// go out in rounds until the device sets its done flag, which the host polls once
+// a round: on the stream in FP64 and in a plan's first run, from hipGraphs in the
+// FP32 runs after it (plan_run).  (A persistent
 // kernel with a grid barrier per sweep measured slower on MI355X: the
 // agent-scope fence each workgroup needs to publish its writes across the
 // eight XCD L2s costs ~36 ns per workgroup, ~19 us per barrier at 512

@@ -92,7 +92,7 @@ def test_solve_returns_the_hosts_order(case):
 
 @pytest.mark.parametrize("rows,cols,src", [(1000, 901, [450123]), (1024, 900, [3, 921599, 400000])])
 def test_large_solve_orders_on_the_device(rows, cols, src):
-    """From 900,000 vertices the plan's own rings give the order."""
+    """Meshes of 0.9M vertices and more, rings of about a thousand."""
     mesh = P.che(*G.height_field_rect(rows, cols, 12))
     order = mesh.compute_toplesets(src)[1]
     d, got, _ = P.ptp(mesh, src, precision=L.PREC_F32, device_setup=True)
